@@ -123,6 +123,7 @@ struct LayerDev {
     const uint16_t* dn_d = nullptr;   // Q6_K down: its fp16 d stream (inside the dn allocation)
     float *gate_b = nullptr, *up_b = nullptr, *down_b = nullptr;
     float *router_w = nullptr, *router_b = nullptr, *norm_w = nullptr;
+    float* router_t = nullptr;  // router_w transposed for the batched router (max_tokens > 1)
     int gu_type = 0, down_type = 0;   // GGUF type ids of this layer's gate/up and down tensors
     bool loaded = false;
     bool mfma_exact = false;    // MXFP4 scales all in [32, 254]: the grouped matrix-core path is exact
@@ -273,7 +274,7 @@ int upload(float** dst, float* slot, const float* src, size_t n, hipStream_t s) 
 // per layer, which keeps their address translations warm.
 size_t align64(size_t n) { return (n + 63) / 64 * 64; }
 struct ParamSlots {
-    size_t router_w, norm_w, router_b, gate_b, up_b, down_b, per_layer;
+    size_t router_w, norm_w, router_b, gate_b, up_b, down_b, router_t, per_layer;
 };
 ParamSlots param_slots(const cpb_moe_cfg& c) {
     const size_t ne = c.n_expert, d = c.d, ff = c.d_ff;
@@ -285,6 +286,7 @@ ParamSlots param_slots(const cpb_moe_cfg& c) {
     p.gate_b = o; o += align64(ne * ff);
     p.up_b = o; o += align64(ne * ff);
     p.down_b = o; o += align64(ne * d);
+    p.router_t = o; o += c.max_tokens > 1 ? align64(cpb::router_t_rows(c.n_expert) * d) : 0;
     p.per_layer = o;
     return p;
 }
@@ -581,6 +583,11 @@ int cpb_moe_load_layer_typed(cpb_moe_t* h, int layer, int gate_type, int up_type
             return r;
     }
     if ((r = upload(&L.router_w, base + ps.router_w, router_w, ne * d, h->stream))) return r;
+    if (c.max_tokens > 1) {
+        L.router_t = base + ps.router_t;
+        if (cpb::launch_router_transpose(L.router_w, L.router_t, c.n_expert, c.d, h->stream))
+            return fail(CPB_ENODEV, "router transpose launch failed");
+    }
     if ((r = upload(&L.norm_w, base + ps.norm_w, norm_w, d, h->stream))) return r;
     HIP_OK(hipStreamSynchronize(h->stream));
     if (h->mx) {
@@ -601,7 +608,7 @@ static int layer_grouped(cpb_moe_t* h, int layer, float* d_x, int n_tok, int app
     const auto& c = h->cfg;
     const LayerDev& L = h->layers[layer];
     cpb::GroupedArgs g{};
-    g.norm_w = L.norm_w; g.router_w = L.router_w; g.router_b = L.router_b;
+    g.norm_w = L.norm_w; g.router_w = L.router_w; g.router_t = L.router_t; g.router_b = L.router_b;
     g.gu = L.gu; g.dn = L.dn; g.dn_d = L.dn_d; g.gate_b = L.gate_b; g.up_b = L.up_b; g.down_b = L.down_b;
     g.n_tok = n_tok; g.d = c.d; g.dff = c.d_ff; g.ne = c.n_expert; g.k = c.top_k; g.nb = h->nb; g.nbf = h->nbf;
     g.parts_gu = h->parts_gu; g.parts_dn = h->parts_dn;

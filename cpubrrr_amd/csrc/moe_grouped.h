@@ -12,6 +12,7 @@ struct GroupedArgs {
     // layer
     const float* norm_w;
     const float* router_w;
+    const float* router_t;     // router_w transposed (launch_router_transpose)
     const float* router_b;
     const u32x4* gu;           // decode stream layouts (moe_mx.hip), read as MFMA operands
     const u32x4* dn;
@@ -54,6 +55,10 @@ struct GroupedArgs {
     int32_t* gu_sums;          // MXFP4 [n_tok*k][2][dff][nb]; Q4_K [n_tok*k][2][dff][d/256][2]
     int32_t* dn_sums;          // MXFP4 [n_tok*k][d][nbf]; Q4_K [..][d][dff/256][2]; Q6_K [..][d][dff/256]
 };
+
+// Rows of the transposed router copy: n_expert up to whole 16-expert groups.
+CPB_DEV_HOST_INLINE int router_t_rows(int ne) { return (ne + 15) / 16 * 16; }
+int launch_router_transpose(const float* w, float* out, int ne, int d, hipStream_t s);
 
 // XCD-aware work order of the grouped GEMMs.  Work item w = (row group
 // w / ntiles, token tile w % ntiles); the workgroups of a launch are dealt to

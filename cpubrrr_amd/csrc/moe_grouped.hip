@@ -41,11 +41,14 @@
 #include "select.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace cpb {
 
 typedef int v8i_g __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+
+typedef __attribute__((address_space(3))) void lds_void_g;
 
 constexpr int kImg = 64;          // image bytes per 32-block
 
@@ -216,6 +219,157 @@ __global__ __launch_bounds__(64) void k_router_exact(GroupedArgs a) {
     }
 }
 
+// The same for batches that leave most of the chip idle, where a chain's
+// length is the kernel's time: workgroup = 16 experts x 4 tokens, whose 64
+// chains are wave 0's lanes (lane 16 r + i: expert 16 ex + i, token 4 ty + r).
+// Wave 0 only adds; four producer waves form the products a chunk of 128 steps
+// ahead, in LDS as wave 0 reads them ([4 steps][lane], 16 bytes).  A
+// producer's unit is 16 steps: its lane 16 r + i holds expert i's row at steps
+// 4 r .. 4 r + 3 (one 1 KB load of the transposed copy, nothing twice) and
+// token c >> 2's xn at step 4 r + (c & 3) in lane 16 r + c, which the product
+// takes by a row broadcast (DPP row_newbcast).  Of three LDS buffers one is
+// being summed, one is complete (so that the reads of the next steps cross
+// into it without a wait) and one is being filled: one barrier per chunk.
+// Bound by the chain: 3.0 ns per step here (a lone wave's dependent add alone
+// takes 1.8, a multiply beside it as much again), behind ~5 us of launch and
+// first loads.  3 tokens x 32 experts x 2880 steps 23.4 -> 14.0 us, 512 tokens
+// 26.5 -> 17.1, 11 tokens x 128 experts x 2048 17.3 -> 11.5 us against
+// k_router_exact.  Every lane reading its own 16 bytes of both operands
+// instead (no exchange) was bound by the L1: four lanes in four read the same.
+constexpr int kPcChunk = 128, kPcProducers = 2, kPcAhead = 6;      // chunks requested ahead
+constexpr int kPcQ = kPcChunk / 4;                // 16-byte units of a chain's chunk
+template <int S>
+CPB_DEV float row_bcast(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + S, 0xf, 0xf, true));
+}
+__global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(GroupedArgs a) {
+    constexpr int UP = kPcChunk / 16 / kPcProducers;   // a producer's units per chunk
+    static_assert(kPcAhead % 3 == 0, "the register sets and the LDS buffers turn together");
+    __shared__ __align__(16) f32x4 prod[3][kPcQ][64];
+    const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6)), d = a.d, nt = a.n_tok, ne = a.ne;
+    const int i = lane & 15, r = lane >> 4, e = blockIdx.x * 16 + i, t = blockIdx.y * 4 + r;
+    // whole rounds of the register sets (the barriers of every wave; chunks past
+    // the row's end are formed from other values or zeros and not summed)
+    const int nch = (d + kPcAhead * kPcChunk - 1) / (kPcAhead * kPcChunk) * kPcAhead;
+    if (w) {
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(a.xn, (uint32_t)((size_t)nt * d * 4));
+        const __amdgpu_buffer_rsrc_t rw = buf_rsrc(a.router_t, (uint32_t)((size_t)router_t_rows(ne) * d * 4));
+        const uint32_t u0 = UP * (w - 1);         // units u0 .. of every chunk
+        const uint32_t wo = (uint32_t)(blockIdx.x * 16 * d) * 4 + u0 * 1024 + lane * 16;
+        const int tx = blockIdx.y * 4 + (i >> 2);
+        const uint32_t xo = tx < nt ? (uint32_t)tx * d * 4 + u0 * 64 + (4 * r + (i & 3)) * 4 : kOffNone;
+        f32x4 wv[kPcAhead][UP];
+        float xv[kPcAhead][UP];
+        auto load = [&](int s, int ch) {
+#pragma unroll
+            for (int u = 0; u < UP; u++) {
+                wv[s][u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo + u * 1024, (uint32_t)ch * (kPcChunk * 64), 0));
+                xv[s][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, xo + u * 64, (uint32_t)ch * (kPcChunk * 4), 0));
+            }
+            __builtin_amdgcn_sched_barrier(0);    // one order of requests everywhere: exact waits
+        };
+        auto emit = [&](int s, int buf) {         // the chunk in register set s
+#pragma unroll
+            for (int u = 0; u < UP; u++) {
+                auto token = [&](auto T) {
+                    constexpr int k = decltype(T)::value;
+                    prod[buf][4 * (u0 + u) + r][16 * k + i] =
+                        f32x4{__fmul_rn(wv[s][u][0], row_bcast<4 * k>(xv[s][u])), __fmul_rn(wv[s][u][1], row_bcast<4 * k + 1>(xv[s][u])),
+                              __fmul_rn(wv[s][u][2], row_bcast<4 * k + 2>(xv[s][u])), __fmul_rn(wv[s][u][3], row_bcast<4 * k + 3>(xv[s][u]))};
+                };
+                token(std::integral_constant<int, 0>{});
+                token(std::integral_constant<int, 1>{});
+                token(std::integral_constant<int, 2>{});
+                token(std::integral_constant<int, 3>{});
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int s = 0; s < kPcAhead; s++) load(s, s);
+        emit(0, 0);
+        load(0, kPcAhead);
+        emit(1, 1);
+        load(1, kPcAhead + 1);
+        for (int k = 0; k < nch; k += kPcAhead) {
+#pragma unroll
+            for (int j = 0; j < kPcAhead; j++) {
+                // the products written so far, and nothing else, before the barrier
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                __builtin_amdgcn_s_barrier();     // chunk k + j - 1 is summed, its buffer free
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                emit((j + 2) % kPcAhead, (j + 2) % 3);            // chunk k + j + 2
+                load((j + 2) % kPcAhead, k + j + 2 + kPcAhead);
+            }
+        }
+        return;
+    }
+    // a chunk's reads are waited for before its sums, so the barrier after them
+    // needs no wait of its own (reads of the next, complete chunk stay in flight)
+    auto arrive = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    };
+    float acc = (a.router_b && e < ne) ? a.router_b[e] : 0.0f;
+    const int nb = d / 32;                        // blocks of 8 units (d % 32 == 0), 4 per chunk
+    f32x4 v[8];
+    auto block = [&](const f32x4* nx) {           // sums the 8 units in v, reads the next 8
+#pragma unroll
+        for (int h = 0; h < 8; h += 4) {
+            asm volatile("" : "+v"(v[h + 3]));    // one wait for the four units
+#pragma unroll
+            for (int u = h; u < h + 4; u++) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) acc = __fadd_rn(acc, v[u][c]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = h; u < h + 4; u++) v[u] = nx[u * 64];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // block m's successor in buffer j: this chunk's, or the first of the next chunk, which is complete
+    auto next = [&](int j, int m) { return m < 3 ? &prod[j][8 * (m + 1)][lane] : &prod[(j + 1) % 3][0][lane]; };
+    int k = 0;
+    arrive();
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = prod[0][u][lane];
+    for (; 4 * (k + 3) <= nb; k += 3) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) block(next(j, m));
+            arrive();                             // of the next chunk
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            if (4 * (k + j) + m < nb) block(next(j, m));
+        if (k + j + 1 < nch) arrive();
+    }
+    for (k += 4; k < nch; k++) arrive();          // the producers' last rounds
+    if (t < nt && e < ne) {
+        a.lstar[(size_t)t * ne + e] = (double)acc;
+        a.lbound[(size_t)t * ne + e] = 0.0;
+    }
+}
+
+// router_w [ne][d] -> router_t [router_t_rows(ne) / 16][d / 4][16][4] (load time; rows past ne zero)
+__global__ __launch_bounds__(256) void k_router_transpose(const float* __restrict__ w, float* __restrict__ out, int ne, int d) {
+    const int i = blockIdx.x * 256 + threadIdx.x;                    // 16-byte unit of the copy
+    if (i >= router_t_rows(ne) * (d / 4)) return;
+    const int j4 = i / 16 % (d / 4), e = i / (16 * (d / 4)) * 16 + i % 16;
+    ((float4*)out)[i] = e < ne ? ((const float4*)w)[(size_t)e * (d / 4) + j4] : float4{0, 0, 0, 0};
+}
+int launch_router_transpose(const float* w, float* out, int ne, int d, hipStream_t s) {
+    hipLaunchKernelGGL(k_router_transpose, dim3((router_t_rows(ne) * (d / 4) + 255) / 256), dim3(256), 0, s, w, out, ne, d);
+    return hipGetLastError() == hipSuccess ? 0 : -19;
+}
+
 
 // ---- 3. top-k + softmax, one wavefront per token (the decode kernels'
 // selection code; on the exact logits of k_router_exact its intervals are
@@ -342,7 +496,6 @@ constexpr int kGuThreads = 256, kDnThreads = 512;
 // fetches the chunk the swizzled layout puts there (token h*16 + L/4 of the
 // block, chunk (L & 3) ^ swz(token)); the scales take 8 instructions of 64
 // (the last half past block 14 reads nothing).
-typedef __attribute__((address_space(3))) void lds_void_g;
 struct DmaPlan {
     __amdgpu_buffer_rsrc_t ri, rs;
     uint32_t vbase0, vbase1, sbase;  // bytes: block 0 of the lane's chunk in token half 0 / 1, its scale
@@ -721,8 +874,11 @@ int launch_grouped_layer(const GroupedArgs& a, bool trace, hipStream_t s, const 
     } else {
         launch(k_prep_batch, dim3(nt), dim3(256), sizeof(float) * (2 * a.d + 64), s, a);
     }
-    // one thread per kRouteC elements, whole waves (the decode route's element waves)
-    launch(k_router_exact, dim3((a.ne + 7) / 8, (nt + 7) / 8), dim3(64), 0, s, a);
+    const int et = router_t_rows(a.ne) / 16, rt = (nt + 3) / 4;
+    // one workgroup of 96 KB LDS per CU: a second round would cost what
+    // k_router_exact takes (777 tokens x 128 experts: 27 us there)
+    if (et * rt <= 256) launch(k_router_exact_small, dim3(et, rt), dim3(64 * (1 + kPcProducers)), 0, s, a);
+    else launch(k_router_exact, dim3((a.ne + 7) / 8, (nt + 7) / 8), dim3(64), 0, s, a);
     launch(k_select_batch, dim3(nt), dim3(64), select_lds_bytes(a.ne, a.d, kExactGroupWide), s, a);
     launch(k_group_scan, dim3(1), dim3(1024), 0, s, a);
     if (a.kq) {

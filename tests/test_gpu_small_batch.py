@@ -1,0 +1,39 @@
+"""GPU parity of the batched (n_tok > 1) path at the sizes where its kernels for
+small batches begin and end: few tokens, expert counts that are no whole
+groups, rows that are no whole chunks, and both sides of each size rule.  The
+expected outputs are grouped_ref's: the reference's combine, with the
+reference's serial fp32 logits, of per-token decode's expert rows."""
+import numpy as np
+import pytest
+
+from cpubrrr_amd import MoeBlock, MoeConfig, synth
+from tests.grouped_ref import BatchCheck, grouped_expect
+
+pytestmark = pytest.mark.gpu
+
+
+def check(L, cfg, X, family):
+    with MoeBlock(cfg) as blk:
+        blk.load_layer(0, L)
+        Y, _ = blk.forward(0, X)
+        bc = BatchCheck()
+        for i in range(X.shape[0]):
+            _, tr = blk.forward(0, X[i], trace=True)
+            ye, _, _ = grouped_expect(L, X[i], tr, family)
+            bc.add(Y[i], ye, X[i], (i,))
+        bc.done()
+
+
+@pytest.mark.parametrize("d,dff,ne,k,n_tok", [
+    (96, 96, 2, 2, 2),          # one block of the router's chain, fewer experts than a group
+    (416, 64, 20, 4, 3),        # 13 blocks, 20 experts
+    (3840, 64, 33, 3, 5),       # the longest row, 33 experts
+    (1088, 96, 16, 1, 17),
+    (448, 64, 128, 4, 128),     # the last size of the small batch's router kernel
+    (448, 64, 128, 4, 129),     # the first of the other
+])
+def test_mxfp4_small_batches(gpu, d, dff, ne, k, n_tok):
+    print(f"case small batch d={d} dff={dff} ne={ne} k={k} n_tok={n_tok}", flush=True)
+    L = synth.gptoss_layer(d, dff, ne, k, seed=21, zipf=1.1)
+    X = np.stack([synth.token(d, 21, i) for i in range(n_tok)])
+    check(L, MoeConfig.gptoss(d=d, n_expert=ne, top_k=k, d_ff=dff, max_tokens=n_tok), X, "gptoss")
