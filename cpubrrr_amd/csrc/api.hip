@@ -488,7 +488,7 @@ int cpb_moe_create(const cpb_moe_cfg* cfg, int device, cpb_moe_t** out) {
             (r = dmalloc(&h->g_lstar, T * ne)) ||
             (r = dmalloc(&h->g_lbound, T * ne)) || (r = dmalloc(&h->g_logits, T * ne)) || (r = dmalloc(&h->g_ids, np)) ||
             (r = dmalloc(&h->g_wts, np)) || (r = dmalloc(&h->g_fallback, T)) || (r = dmalloc(&h->g_sorted, np)) ||
-            (r = dmalloc(&h->g_tiles, np / 32 + ne + 1)) || (r = dmalloc(&h->g_ntiles, 1)) ||
+            (r = dmalloc(&h->g_tiles, cpb::grouped_max_tiles(np, ne, cpb::kFewTile))) || (r = dmalloc(&h->g_ntiles, 1)) ||
             (r = dmalloc(&h->g_hq, np * ff)) || (r = dmalloc(&h->g_hsb, np * nbf)) || (r = dmalloc(&h->g_dnout, np * d)))
             return bail(r);
         if (h->mx && ((r = dmalloc(&h->g_ximg, T * nb * 64)) || (r = dmalloc(&h->g_himg, np * nbf * 64)))) return bail(r);
@@ -614,7 +614,8 @@ static int layer_grouped(cpb_moe_t* h, int layer, float* d_x, int n_tok, int app
     g.parts_gu = h->parts_gu; g.parts_dn = h->parts_dn;
     g.norm = c.norm; g.norm_nt = c.norm_nt; g.apply_norm = apply_norm;
     g.eps = c.rms_eps; g.alpha = c.alpha; g.limit = c.limit;
-    g.max_tiles = n_tok * c.top_k / 32 + c.n_expert + 1;
+    g.tile = h->mx || gu_sums ? 32 : cpb::kq_tile(n_tok * c.top_k, c.n_expert, c.d_ff);
+    g.max_tiles = cpb::grouped_max_tiles(n_tok * c.top_k, c.n_expert, g.tile);
     g.x = d_x; g.xn = h->g_xn; g.inv = h->g_inv; g.xq = h->g_xq; g.xsb = h->g_xsb; g.ximg = h->g_ximg;
     g.lstar = h->g_lstar; g.lbound = h->g_lbound; g.logits = h->g_logits; g.ids = h->g_ids; g.wts = h->g_wts;
     g.fallback = h->g_fallback; g.sorted = h->g_sorted; g.tiles = h->g_tiles; g.ntiles = h->g_ntiles;

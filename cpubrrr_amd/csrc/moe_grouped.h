@@ -24,7 +24,8 @@ struct GroupedArgs {
     int n_tok, d, dff, ne, k, nb, nbf, parts_gu, parts_dn;
     int norm, norm_nt, apply_norm;
     float eps, alpha, limit;
-    int max_tiles;             // grid bound of the expert GEMMs: n_tok*k/32 + ne
+    int tile;                  // pairs per tile: 32, or kFewTile (k-quant small batches)
+    int max_tiles;             // grid bound of the expert GEMMs (grouped_max_tiles)
     // activations (device)
     float* x;                  // [n_tok][d] residual, updated in place
     float* xn;                 // [n_tok][d]
@@ -55,6 +56,14 @@ struct GroupedArgs {
     int32_t* gu_sums;          // MXFP4 [n_tok*k][2][dff][nb]; Q4_K [n_tok*k][2][dff][d/256][2]
     int32_t* dn_sums;          // MXFP4 [n_tok*k][d][nbf]; Q4_K [..][d][dff/256][2]; Q6_K [..][d][dff/256]
 };
+
+// Most tiles of `tile` pairs that np pairs over ne experts can make: a used
+// expert's last tile may be short.
+CPB_DEV_HOST_INLINE int grouped_max_tiles(int np, int ne, int tile) { return np / tile + (np < ne ? np : ne); }
+// k-quant batches: pairs per tile of the few-token kernels, and the tile size
+// for np pairs over ne experts (kFewTile or 32)
+constexpr int kFewTile = 8;
+int kq_tile(int np, int ne, int dff);
 
 // Rows of the transposed router copy: n_expert up to whole 16-expert groups.
 CPB_DEV_HOST_INLINE int router_t_rows(int ne) { return (ne + 15) / 16 * 16; }

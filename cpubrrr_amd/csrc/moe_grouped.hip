@@ -400,7 +400,7 @@ __global__ __launch_bounds__(64) void k_select_batch(GroupedArgs a) {
 // One workgroup: each pair takes its place among its expert's pairs from an
 // LDS counter (arrival order: any order serves, a pair's outputs do not
 // depend on its tile or on the other pairs there), then the exclusive prefix
-// of the counts (pairs and 32-pair tiles), each pair written at its expert's
+// of the counts (pairs and tiles of a.tile pairs), each pair written at its expert's
 // offset + its place, and the tile list.
 constexpr int kScanPer = 16;                   // pairs per thread held in registers
 // One workgroup; the caller's config check bounds n_expert <= 256 (the LDS
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(1024) void k_group_scan(GroupedArgs a) {
         for (int base = 0; base < ne; base += 64) {
             const int e = base + lane;
             const int c = e < ne ? cnt_l[e] : 0;
-            const int tl = (c + 31) / 32;
+            const int tl = (c + a.tile - 1) / a.tile;
             int ic = c, it = tl;
 #pragma unroll
             for (int s2 = 1; s2 < 64; s2 <<= 1) {
@@ -445,8 +445,8 @@ __global__ __launch_bounds__(1024) void k_group_scan(GroupedArgs a) {
     for (int u = 0; u < kScanPer; u++)
         if (ex[u] >= 0) a.sorted[off_l[ex[u]] + rk[u]] = tid + u * 1024;
     for (int e = w; e < ne; e += 16) {
-        const int c = cnt_l[e], nt = (c + 31) / 32;
-        for (int j = lane; j < nt; j += 64) a.tiles[toff_l[e] + j] = int4{e, off_l[e] + 32 * j, min(32, c - 32 * j), 0};
+        const int c = cnt_l[e], nt = (c + a.tile - 1) / a.tile;
+        for (int j = lane; j < nt; j += 64) a.tiles[toff_l[e] + j] = int4{e, off_l[e] + a.tile * j, min(a.tile, c - a.tile * j), 0};
     }
 }
 

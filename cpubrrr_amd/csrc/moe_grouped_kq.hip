@@ -32,6 +32,7 @@
 #include "moe_common.h"
 #include "moe_grouped.h"
 #include "moe_kq.h"
+#include "kq_dev.h"
 #include "route_dev.h"
 
 #include <algorithm>
@@ -531,12 +532,147 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
 }
 
+// ---- small batches: few tokens per expert ----
+// A 32-token matrix-core tile is mostly padding when an expert has one or two
+// tokens, and its kernels' prologue and LDS traffic then outweigh the weight
+// stream.  These take tiles of up to kFewTile pairs the way batch-1 decode
+// takes its one token (moe_kq.hip: a lane's (row, superblock) units in
+// registers, its term with the reference's operations, terms added in
+// superblock order), each token of the tile against the same registers.  Bound
+// by the weight stream at the sizes that take them (kq_tile).
+
+// gate/up + SiLU * up: workgroup = (tile, 16 rows), a wave per two superblocks
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_gateup_kq_few(GroupedArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int nsb = a.d / 256, T = a.dff / 16;
+    int tile, t;
+    if (!grouped_item(uniform(*a.ntiles), T, &tile, &t)) return;
+    const int4 tl = a.tiles[tile];
+    const int e = uniform(tl.x), start = uniform(tl.y), cnt = uniform(tl.z);
+    const int lane = threadIdx.x & 63, q = uniform((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
+    int8_t* xl = (int8_t*)smem;                                  // [kFewTile][nsb][kXsPad]
+    int32_t* xsl = (int32_t*)(smem + kFewTile * nsb * kXsPad);   // [kFewTile][nsb * 8]
+    float* ysl = (float*)(xsl + kFewTile * nsb * 8);             // [kFewTile][nsb]
+    float* part = ysl + kFewTile * nsb;                          // [kFewTile][nsb][32]
+    // weights first: they need the expert only
+    const int s = 2 * q + (lane >> 5), r = lane & 31;
+    const bool live = s < nsb;
+    const u32x4* wp = a.gu + ((((size_t)e * T + t) * nsb + (live ? s : 0)) * kQ4Units) * 32 + r;
+    u32x4 u[kQ4Units];
+#pragma unroll
+    for (int k = 0; k < kQ4Units; k++) u[k] = __builtin_nontemporal_load(wp + k * 32);
+    // wave q brings tokens q, q + nw, ..
+    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(a.xq, (uint32_t)((size_t)a.n_tok * a.d));
+    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(a.xsum, (uint32_t)((size_t)a.n_tok * (a.d / 32) * 4));
+    const __amdgpu_buffer_rsrc_t ry = buf_rsrc(a.xsb, (uint32_t)((size_t)a.n_tok * nsb * 4));
+    for (int ti = q; ti < cnt; ti += nw) {
+        const uint32_t tok = (uint32_t)(uniform(a.sorted[start + ti]) / a.k);
+        for (int i = lane; i < a.d / 16; i += 64)
+            *(u32x4*)(xl + (ti * nsb + i / 16) * kXsPad + (i % 16) * 16) = __builtin_amdgcn_raw_buffer_load_b128(rx, tok * a.d + i * 16, 0, 0);
+        for (int i = lane; i < nsb * 8; i += 64) xsl[ti * nsb * 8 + i] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, (tok * (nsb * 8) + i) * 4, 0, 0);
+        if (lane < nsb) ysl[ti * nsb + lane] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ry, (tok * nsb + lane) * 4, 0, 0));
+    }
+    __syncthreads();
+    if (live) {
+        for (int ti = 0; ti < cnt; ti++)
+            part[(ti * nsb + s) * 32 + r] = q4k_term<false>(u, xl + (ti * nsb + s) * kXsPad, xsl + (ti * nsb + s) * 8, ysl[ti * nsb + s], nullptr);
+    }
+    __syncthreads();
+    for (int ti = threadIdx.x >> 5; ti < cnt; ti += blockDim.x >> 5) {
+        float v = 0.0f;                                          // sumf, superblocks in order
+        for (int k = 0; k < nsb; k++) v += part[(ti * nsb + k) * 32 + r];
+        const float up = __shfl_down(v, 16);
+        if (r < 16) a.hbuf[(size_t)a.sorted[start + ti] * a.dff + t * 16 + r] = (v / (1.0f + expf(-v))) * up;   // :416
+    }
+}
+
+// Q8_K of h (into LDS) + down into dnout: workgroup = (tile, 64 rows), a wave per superblock
+static size_t few_down_lds(int dff) {
+    const int nsbf = dff / 256, nch = kFewTile * dff / 32;
+    return (size_t)kFewTile * nsbf * kXsPad + nch * 4 * 4 + kFewTile * nsbf * 4 + (size_t)std::max(kFewTile * nsbf * 64 * 4, nch * 128) + 16;
+}
+template <int TYPE>
+__global__ __launch_bounds__(1024) void k_down_kq_few(GroupedArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int U = TYPE == 12 ? kQ4Units : kQ6Units, SU = TYPE == 12 ? kQ4Units : kQ6StreamUnits;
+    const int RT = 64 / a.k, nsbf = a.dff / 256, T = a.d / RT;
+    int tile, grp;
+    if (!grouped_item(uniform(*a.ntiles), a.d / 64, &tile, &grp)) return;
+    const int4 tl = a.tiles[tile];
+    const int e = uniform(tl.x), start = uniform(tl.y), cnt = uniform(tl.z);
+    const int lane = threadIdx.x & 63, q = uniform((int)(threadIdx.x >> 6));
+    const int cps = a.dff / 32, nch = cnt * cps, hstride = nsbf * kXsPad;
+    int8_t* hql = (int8_t*)smem;                                  // [kFewTile][nsbf][kXsPad]
+    float* cmax = (float*)(smem + kFewTile * hstride);            // [kFewTile * dff / 32]
+    int32_t* h32 = (int32_t*)(cmax + kFewTile * cps);
+    int32_t* h16 = h32 + kFewTile * cps;
+    float* hsl = (float*)(h16 + 2 * kFewTile * cps);              // [kFewTile * nsbf]
+    const int off = (int)((unsigned char*)(hsl + kFewTile * nsbf) - smem);
+    float4* hst = (float4*)(smem + ((off + 15) & ~15));           // h chunks, then the terms [kFewTile][nsbf][64]
+    float* part = (float*)hst;
+    // this thread's chunk of h, then the weights (as the decode kernel: the
+    // Q8_K runs while the weights are in flight)
+    const int c = (int)threadIdx.x;                               // nch <= 64 nsbf
+    float4 hv[8];
+    {
+        const int cl = c < nch ? c : 0;
+        const float4* src = (const float4*)(a.hbuf + (size_t)a.sorted[start + cl / cps] * a.dff + (cl % cps) * 32);
+#pragma unroll
+        for (int k = 0; k < 8; k++) hv[k] = src[k];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int row = grp * 64 + lane;
+    const size_t sbi = ((size_t)e * T + row / RT) * nsbf + q;     // (expert, row tile, superblock)
+    const u32x4* wp = a.dn + sbi * SU * RT + row % RT;
+    u32x4 u[U];
+#pragma unroll
+    for (int k = 0; k < SU; k++) u[k] = __builtin_nontemporal_load(wp + k * RT);
+    if constexpr (TYPE == 14) u[kQ6Units - 1] = u32x4{(uint32_t)__builtin_nontemporal_load(a.dn_d + sbi * RT + row % RT), 0, 0, 0};
+    __builtin_amdgcn_sched_barrier(0);
+    quant_h_chunks(hv, c, nch, cps, hstride, hst, cmax, hql, h32, h16, hsl);
+    for (int ti = 0; ti < cnt; ti++) {
+        const int8_t* xs = hql + ti * hstride + q * kXsPad;
+        const float ys = hsl[ti * nsbf + q];
+        float tv;
+        if constexpr (TYPE == 12) tv = q4k_term<false>(u, xs, h32 + (ti * nsbf + q) * 8, ys, nullptr);
+        else tv = q6k_term<false>(u, xs, h16 + (ti * nsbf + q) * 16, ys, nullptr);
+        part[(ti * nsbf + q) * 64 + lane] = tv;
+    }
+    __syncthreads();
+    for (int ti = q; ti < cnt; ti += nsbf) {
+        float v = 0.0f;
+        for (int k = 0; k < nsbf; k++) v += part[(ti * nsbf + k) * 64 + lane];
+        a.dnout[(size_t)a.sorted[start + ti] * a.d + row] = v + (a.down_b ? a.down_b[(size_t)e * a.d + row] : 0.0f);
+    }
+}
+
+// Up to four pairs per expert on average the few-token kernels are faster
+// (whole layer, 128 experts top-8; d 2048, d_ff 768, Q6_K down: 4 tokens 60.1
+// against 82.4 us, 64 tokens 140 against 169, 128 tokens 191 against 172; d
+// 4096, d_ff 1536, Q4_K down: 16 tokens 233 against 311 us, 64 tokens 422
+// against 436, 128 tokens 654 against 450), and where the down kernel's LDS
+// leaves room for two workgroups per CU (d_ff <= 1536).
+int kq_tile(int np, int ne, int dff) {
+    return np <= 4 * ne && few_down_lds(dff) <= 76 * 1024 ? kFewTile : 32;
+}
+
 int launch_prep_kq(const GroupedArgs& a, hipStream_t s) {
     launch(k_prep_batch_kq, dim3(a.n_tok), dim3(256), sizeof(float) * (2 * a.d + 64), s, a);
     return hipGetLastError() == hipSuccess ? 0 : -19;
 }
 
 int launch_kq_gemms(const GroupedArgs& a, bool trace, hipStream_t s, const LaunchEvents* ev) {
+    if (a.tile == kFewTile) {
+        const int nsb = a.d / 256, nsbf = a.dff / 256;
+        const int ngf = a.max_tiles * (a.dff / 16), ndf = a.max_tiles * (a.d / 64);
+        const size_t lgu = (size_t)kFewTile * nsb * (kXsPad + 32 + 4 + 128), ldn = few_down_lds(a.dff);
+        if (ev) armed_events() = ev[0];
+        launch(k_gateup_kq_few, dim3((ngf + 7) / 8 * 8), dim3(64 * ((nsb + 1) / 2)), lgu, s, a);
+        if (ev) armed_events() = ev[1];
+        if (a.down_type == 12) launch(k_down_kq_few<12>, dim3((ndf + 7) / 8 * 8), dim3(64 * nsbf), ldn, s, a);
+        else launch(k_down_kq_few<14>, dim3((ndf + 7) / 8 * 8), dim3(64 * nsbf), ldn, s, a);
+        return hipGetLastError() == hipSuccess ? 0 : -19;
+    }
     const int ngu = a.max_tiles * ((a.dff / 32 + 1) / 2), ndn = a.max_tiles * ((a.d / 32 + 3) / 4);
     const dim3 ggu((ngu + 7) / 8 * 8), gdn((ndn + 7) / 8 * 8);
     const int np = a.n_tok * a.k, nq = np * (a.dff / 256);

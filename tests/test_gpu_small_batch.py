@@ -37,3 +37,21 @@ def test_mxfp4_small_batches(gpu, d, dff, ne, k, n_tok):
     L = synth.gptoss_layer(d, dff, ne, k, seed=21, zipf=1.1)
     X = np.stack([synth.token(d, 21, i) for i in range(n_tok)])
     check(L, MoeConfig.gptoss(d=d, n_expert=ne, top_k=k, d_ff=dff, max_tokens=n_tok), X, "gptoss")
+
+
+@pytest.mark.parametrize("d,dff,ne,k,n_tok,down,same", [
+    (256, 256, 8, 2, 3, 14, False),         # one superblock in each matrix
+    (512, 512, 16, 8, 5, 12, False),
+    (768, 768, 20, 1, 7, 14, False),        # an odd superblock count, top-1
+    # one token nine times: an expert's second tile.  (Copies of a token share its expf ulps, so
+    # BatchCheck's share of bit-exact tokens, taken from ten tokens on, would say nothing.)
+    (512, 1536, 16, 4, 9, 12, True),
+    (1280, 768, 16, 4, 16, 14, False),      # four pairs per expert: the last size of the few-token kernels
+    (1280, 768, 16, 4, 17, 14, False),      # the first of the matrix-core tiles
+    (512, 2048, 16, 2, 4, 14, False),       # d_ff beyond the few-token down kernel
+])
+def test_kq_small_batches(gpu, d, dff, ne, k, n_tok, down, same):
+    print(f"case kq small batch d={d} dff={dff} ne={ne} k={k} n_tok={n_tok} down={down}", flush=True)
+    L = synth.qwen_layer(d, dff, ne, k, seed=22, down_type=down)
+    X = np.stack([synth.token(d, 22, 0 if same else i) for i in range(n_tok)])
+    check(L, MoeConfig.qwen3(d=d, n_expert=ne, top_k=k, d_ff=dff, max_tokens=n_tok, down_type=down), X, "qwen")
