@@ -152,11 +152,10 @@ struct cpb_moe {
     size_t staging_size = 0;
     // grouped (n_tok > 1) MXFP4 path: per-token and per-pair scratch
     bool grouped = false;
-    float *g_inv = nullptr, *g_xn = nullptr, *g_xsb = nullptr, *g_logits = nullptr, *g_wts = nullptr, *g_hsb = nullptr, *g_dnout = nullptr;
+    float *g_xn = nullptr, *g_xsb = nullptr, *g_logits = nullptr, *g_wts = nullptr, *g_hsb = nullptr, *g_dnout = nullptr;
     int8_t *g_xq = nullptr, *g_hq = nullptr;
     uint8_t *g_ximg = nullptr, *g_himg = nullptr;
-    double *g_lstar = nullptr, *g_lbound = nullptr;
-    int32_t *g_ids = nullptr, *g_fallback = nullptr, *g_sorted = nullptr, *g_ntiles = nullptr;
+    int32_t *g_ids = nullptr, *g_sorted = nullptr, *g_ntiles = nullptr;
     int32_t *g_xsum = nullptr, *g_hsum = nullptr;   // k-quant grouped path
     float* g_hbuf = nullptr;
     int4* g_tiles = nullptr;
@@ -484,10 +483,9 @@ int cpb_moe_create(const cpb_moe_cfg* cfg, int device, cpb_moe_t** out) {
         // grouped (batched) path: per-token and per-pair buffers; MXFP4 uses
         // the fp8 images, the k-quant path the per-32 sums and fp32 h
         const size_t nb = d / 32, nbf = ff / 32, np = T * k;
-        if ((r = dmalloc(&h->g_xn, T * d)) || (r = dmalloc(&h->g_inv, T)) || (r = dmalloc(&h->g_xq, T * d)) || (r = dmalloc(&h->g_xsb, T * nb)) ||
-            (r = dmalloc(&h->g_lstar, T * ne)) ||
-            (r = dmalloc(&h->g_lbound, T * ne)) || (r = dmalloc(&h->g_logits, T * ne)) || (r = dmalloc(&h->g_ids, np)) ||
-            (r = dmalloc(&h->g_wts, np)) || (r = dmalloc(&h->g_fallback, T)) || (r = dmalloc(&h->g_sorted, np)) ||
+        if ((r = dmalloc(&h->g_xn, T * d)) || (r = dmalloc(&h->g_xq, T * d)) || (r = dmalloc(&h->g_xsb, T * nb)) ||
+            (r = dmalloc(&h->g_logits, T * ne)) || (r = dmalloc(&h->g_ids, np)) ||
+            (r = dmalloc(&h->g_wts, np)) || (r = dmalloc(&h->g_sorted, np)) ||
             (r = dmalloc(&h->g_tiles, cpb::grouped_max_tiles(np, ne, cpb::kFewTile))) || (r = dmalloc(&h->g_ntiles, 1)) ||
             (r = dmalloc(&h->g_hq, np * ff)) || (r = dmalloc(&h->g_hsb, np * nbf)) || (r = dmalloc(&h->g_dnout, np * d)))
             return bail(r);
@@ -616,9 +614,9 @@ static int layer_grouped(cpb_moe_t* h, int layer, float* d_x, int n_tok, int app
     g.eps = c.rms_eps; g.alpha = c.alpha; g.limit = c.limit;
     g.tile = h->mx || gu_sums ? 32 : cpb::kq_tile(n_tok * c.top_k, c.n_expert, c.d_ff);
     g.max_tiles = cpb::grouped_max_tiles(n_tok * c.top_k, c.n_expert, g.tile);
-    g.x = d_x; g.xn = h->g_xn; g.inv = h->g_inv; g.xq = h->g_xq; g.xsb = h->g_xsb; g.ximg = h->g_ximg;
-    g.lstar = h->g_lstar; g.lbound = h->g_lbound; g.logits = h->g_logits; g.ids = h->g_ids; g.wts = h->g_wts;
-    g.fallback = h->g_fallback; g.sorted = h->g_sorted; g.tiles = h->g_tiles; g.ntiles = h->g_ntiles;
+    g.x = d_x; g.xn = h->g_xn; g.xq = h->g_xq; g.xsb = h->g_xsb; g.ximg = h->g_ximg;
+    g.logits = h->g_logits; g.ids = h->g_ids; g.wts = h->g_wts;
+    g.sorted = h->g_sorted; g.tiles = h->g_tiles; g.ntiles = h->g_ntiles;
     g.hq = h->g_hq; g.hsb = h->g_hsb; g.himg = h->g_himg; g.dnout = h->g_dnout;
     g.kq = h->mx ? 0 : 1; g.down_type = L.down_type;
     g.xsum = h->g_xsum; g.hbuf = h->g_hbuf; g.hsum = h->g_hsum;
@@ -867,8 +865,8 @@ void cpb_moe_destroy(cpb_moe_t* h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     clear_graphs(h);
     void* gbufs[] = {h->g_xsum, h->g_hsum, h->g_hbuf,
-                     h->g_inv, h->g_xn, h->g_xsb, h->g_logits, h->g_wts, h->g_hsb, h->g_dnout, h->g_xq, h->g_hq, h->g_ximg,
-                     h->g_himg, h->g_lstar, h->g_lbound, h->g_ids, h->g_fallback, h->g_sorted, h->g_ntiles, h->g_tiles,
+                     h->g_xn, h->g_xsb, h->g_logits, h->g_wts, h->g_hsb, h->g_dnout, h->g_xq, h->g_hq, h->g_ximg,
+                     h->g_himg, h->g_ids, h->g_sorted, h->g_ntiles, h->g_tiles,
                      h->d_special};
     for (void* p : gbufs) (void)hipFree(p);
     for (auto& L : h->layers) free_layer(L);

@@ -29,16 +29,12 @@ struct GroupedArgs {
     // activations (device)
     float* x;                  // [n_tok][d] residual, updated in place
     float* xn;                 // [n_tok][d]
-    float* inv;                // [n_tok] rmsnorm scale (1 without the norm)
     int8_t* xq;                // [n_tok][d]
     float* xsb;                // [n_tok][nb]
     uint8_t* ximg;             // [n_tok][nb][64] fp8 image of xq (MFMA operand)
-    double* lstar;             // [n_tok][ne]
-    double* lbound;            // [n_tok][ne]
-    float* logits;             // [n_tok][ne]
-    int32_t* ids;              // [n_tok][k]
+    float* logits;             // [n_tok][ne] the reference's fp32 logits
+    int32_t* ids;              // [n_tok][k] (batches beyond k_select_group)
     float* wts;                // [n_tok][k]
-    int32_t* fallback;         // [n_tok]
     int32_t* sorted;           // [n_tok*k] pair ids (t*k + slot), grouped by expert (any order within one)
     int4* tiles;               // [max_tiles] {expert, first sorted index, count, 0}
     int32_t* ntiles;           // [1]

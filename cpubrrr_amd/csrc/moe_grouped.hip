@@ -61,7 +61,6 @@ __global__ __launch_bounds__(256) void k_prep_batch(GroupedArgs a) {
     float* xnl = xs + d;
     float* scratch = xnl + d;
     norm_into(a.x + (size_t)t * d, a.norm_w, d, a.eps, a.norm, a.norm_nt, a.apply_norm, xs, xnl, scratch);
-    if (tid == 0) a.inv[t] = a.apply_norm ? scratch[16] : 1.0f;
     // Q8 per 32-block (engine_gpt2.rs:691-699), four threads per block:
     // thread c owns elements 8p + 4h .. +3 and 16 + 8p + 4h .. +3 (p = c >> 1,
     // h = c & 1), so its share of xq is two whole dwords and its share of the
@@ -146,9 +145,8 @@ __global__ __launch_bounds__(256) void k_prep_batch(GroupedArgs a) {
 // the products one step ahead of the adds.  The 8 tokens' xn and the 8
 // experts' router rows stream through LDS in chunks of kChainChunk (the next
 // chunk requested into registers while the current one is summed).  The
-// logit goes to lstar with a zero lbound: the selection then ranks exact
-// values and never needs its exact path, and the weights are the softmax of
-// the reference's own fp32 logits.
+// selection ranks these values, and the weights are the softmax of the
+// reference's own fp32 logits.
 constexpr int kChainChunk = 128;
 constexpr int kChainStride = kChainChunk + 4;     // floats per LDS row (spreads the 8 rows over the banks)
 __global__ __launch_bounds__(64) void k_router_exact(GroupedArgs a) {
@@ -213,10 +211,7 @@ __global__ __launch_bounds__(64) void k_router_exact(GroupedArgs a) {
             put(buf ^ 1, xr, wr);
         }
     }
-    if (t < nt && e < ne) {
-        a.lstar[(size_t)t * ne + e] = (double)acc;
-        a.lbound[(size_t)t * ne + e] = 0.0;
-    }
+    if (t < nt && e < ne) a.logits[(size_t)t * ne + e] = acc;
 }
 
 // The same for batches that leave most of the chip idle, where a chain's
@@ -352,10 +347,7 @@ __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(
         if (k + j + 1 < nch) arrive();
     }
     for (k += 4; k < nch; k++) arrive();          // the producers' last rounds
-    if (t < nt && e < ne) {
-        a.lstar[(size_t)t * ne + e] = (double)acc;
-        a.lbound[(size_t)t * ne + e] = 0.0;
-    }
+    if (t < nt && e < ne) a.logits[(size_t)t * ne + e] = acc;
 }
 
 // router_w [ne][d] -> router_t [router_t_rows(ne) / 16][d / 4][16][4] (load time; rows past ne zero)
@@ -371,55 +363,85 @@ int launch_router_transpose(const float* w, float* out, int ne, int d, hipStream
 }
 
 
-// ---- 3. top-k + softmax, one wavefront per token (the decode kernels'
-// selection code; on the exact logits of k_router_exact its intervals are
-// points, so the ids are the reference's and the weights the softmax of the
-// reference's fp32 logits) ----
-__global__ __launch_bounds__(64) void k_select_batch(GroupedArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ Selection sel;
-    const int lane = threadIdx.x, t = blockIdx.x;
-    SelectIn si{};
-    si.lstar = a.lstar + (size_t)t * a.ne;
-    si.lbound = a.lbound + (size_t)t * a.ne;
-    si.router_w = a.router_w;
-    si.router_b = a.router_b;
-    si.xn = a.xn + (size_t)t * a.d;
-    si.ne = a.ne; si.k = a.k; si.d = a.d;
-    si.logits = a.logits + (size_t)t * a.ne;      // written by every workgroup: one per token
-    select_topk_wave<8, 4>(si, smem, &sel, true);
-    if (lane < a.k) {
-        const int e = sel.ids[lane];
-        a.ids[(size_t)t * a.k + lane] = e;
-        a.wts[(size_t)t * a.k + lane] = sel.wts[lane];
+// ---- 3. top-k + softmax of a token's exact logits, one wavefront ----
+// The reference selects by descending value with the lowest index winning ties
+// (engine_gpt2.rs:852-867 insertion with strict comparisons;
+// engine_qwen2.rs:403-410 stable sort), then takes a softmax over the k
+// selected.  The logits are the reference's own, so the order is exact on
+// them: lane l holds experts l + 64 j as order-preserving 32-bit keys, K
+// rounds of a wave maximum, the lowest index by ballot.  A NaN ranks last (a
+// strict comparison never lets one in), as -inf.
+struct TokenLogits {
+    float v[4];
+};
+CPB_DEV TokenLogits load_logits(const GroupedArgs& a, int t) {
+    TokenLogits l;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int e = (int)(threadIdx.x & 63) + 64 * j;
+        l.v[j] = e < a.ne && t < a.n_tok ? a.logits[(size_t)t * a.ne + e] : 0.0f;
     }
-    if (lane == 0) a.fallback[t] = sel.fallback;
+    return l;
+}
+// rank i's expert in lane i < k (the softmax weights go to a.wts)
+CPB_DEV int select_exact(const GroupedArgs& a, const TokenLogits& l, int t) {
+    const int lane = threadIdx.x & 63, K = a.k;
+    uint32_t key[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float v = l.v[j] + 0.0f;                   // -0 and +0 are equal
+        key[j] = lane + 64 * j < a.ne ? (v == v ? float_key(v) : 1u) : 0u;      // float_key(-inf) > 1
+    }
+    int my_e = 0;
+    uint32_t my_k = 0u;
+    for (int i = 0; i < K; i++) {
+        const uint32_t m = wave_max_u32(max(max(key[0], key[1]), max(key[2], key[3])));
+        int e = 0;
+#pragma unroll
+        for (int j = 3; j >= 0; j--) {
+            const uint64_t b = __ballot(key[j] == m);
+            if (b) e = 64 * j + (int)__builtin_ctzll(b);
+        }
+        if (lane == i) { my_e = e; my_k = m; }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (lane + 64 * j == e) key[j] = 0u;         // taken
+    }
+    const float my_l = my_k > 1u ? key_float(my_k) : -__builtin_inff();
+    // softmax over the k selected, reference order: ex_i = exp(l_i - l_0)
+    // (lane i), then the serial sum ex_0 + ex_1 + ...
+    const float l0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_l), 0));
+    const float ex = expf(my_l - l0);
+    float wsum = 0.0f;
+    for (int i = 0; i < K; i++) wsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ex), i));
+    if (lane < K) a.wts[(size_t)t * K + lane] = ex / wsum;
+    return my_e;
+}
+
+__global__ __launch_bounds__(256) void k_select_batch(GroupedArgs a) {
+    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (t >= a.n_tok) return;
+    const int e = select_exact(a, load_logits(a, t), t);
+    if (lane < a.k) a.ids[(size_t)t * a.k + lane] = e;
 }
 
 // ---- 4. grouping by expert ----
-// One workgroup: each pair takes its place among its expert's pairs from an
-// LDS counter (arrival order: any order serves, a pair's outputs do not
-// depend on its tile or on the other pairs there), then the exclusive prefix
-// of the counts (pairs and tiles of a.tile pairs), each pair written at its expert's
-// offset + its place, and the tile list.
-constexpr int kScanPer = 16;                   // pairs per thread held in registers
-// One workgroup; the caller's config check bounds n_expert <= 256 (the LDS
-// tables) and n_tok * k <= 16384 = kScanPer * 1024 (the pairs per thread).
-__global__ __launch_bounds__(1024) void k_group_scan(GroupedArgs a) {
+// One workgroup of 1024 threads, thread tid holding the experts of pairs tid +
+// 1024 u (u < PER; -1: none): each pair takes its place among its expert's
+// pairs from an LDS counter (arrival order: any order serves, a pair's outputs
+// do not depend on its tile or on the other pairs there), then the exclusive
+// prefix of the counts (pairs and tiles of a.tile pairs), each pair written at
+// its expert's offset + its place, and the tile list.  The caller's config
+// check bounds n_expert <= 256 (the LDS tables).
+template <int PER>
+CPB_DEV void group_pairs(const GroupedArgs& a, const int (&ex)[PER]) {
     __shared__ int cnt_l[256], off_l[256], toff_l[256];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int np = a.n_tok * a.k, ne = a.ne;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, ne = a.ne;
     for (int e = tid; e < ne; e += blockDim.x) cnt_l[e] = 0;
-    // every pair's expert requested before the first wait
-    int ex[kScanPer], rk[kScanPer];
-#pragma unroll
-    for (int u = 0; u < kScanPer; u++) {
-        const int p = tid + u * 1024;
-        ex[u] = p < np ? a.ids[p] : -1;
-    }
+    int rk[PER];
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kScanPer; u++)
+    for (int u = 0; u < PER; u++)
         rk[u] = ex[u] >= 0 ? __hip_atomic_fetch_add(cnt_l + ex[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0;
     __syncthreads();
     if (w == 0) {
@@ -442,12 +464,45 @@ __global__ __launch_bounds__(1024) void k_group_scan(GroupedArgs a) {
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kScanPer; u++)
+    for (int u = 0; u < PER; u++)
         if (ex[u] >= 0) a.sorted[off_l[ex[u]] + rk[u]] = tid + u * 1024;
     for (int e = w; e < ne; e += 16) {
         const int c = cnt_l[e], nt = (c + a.tile - 1) / a.tile;
         for (int j = lane; j < nt; j += 64) a.tiles[toff_l[e] + j] = int4{e, off_l[e] + a.tile * j, min(a.tile, c - a.tile * j), 0};
     }
+}
+// n_tok * k <= 16384 = kScanPer * 1024 (the caller's config check)
+constexpr int kScanPer = 16;                   // pairs per thread held in registers
+__global__ __launch_bounds__(1024) void k_group_scan(GroupedArgs a) {
+    const int np = a.n_tok * a.k;
+    int ex[kScanPer];                          // every pair's expert requested before the first wait
+#pragma unroll
+    for (int u = 0; u < kScanPer; u++) {
+        const int p = (int)threadIdx.x + u * 1024;
+        ex[u] = p < np ? a.ids[p] : -1;
+    }
+    group_pairs<kScanPer>(a, ex);
+}
+// Small batches: selection and grouping in one launch, a wave per kSelTok
+// tokens (16 waves; np <= 1024)
+constexpr int kSelTok = 4, kSelMax = 16 * kSelTok;
+__global__ __launch_bounds__(1024) void k_select_group(GroupedArgs a) {
+    __shared__ int ids_l[kSelMax * 8];
+    const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6)), np = a.n_tok * a.k;
+    TokenLogits l[kSelTok];
+#pragma unroll
+    for (int i = 0; i < kSelTok; i++) l[i] = load_logits(a, w + 16 * i);
+#pragma unroll
+    for (int i = 0; i < kSelTok; i++) {
+        const int t = w + 16 * i;
+        if (t < a.n_tok) {
+            const int e = select_exact(a, l[i], t);
+            if (lane < a.k) ids_l[t * a.k + lane] = e;
+        }
+    }
+    __syncthreads();
+    const int ex[1] = {(int)threadIdx.x < np ? ids_l[threadIdx.x] : -1};
+    group_pairs<1>(a, ex);
 }
 
 // One block of the grouped product: A = 16 raw code bytes (both K halves),
@@ -879,8 +934,12 @@ int launch_grouped_layer(const GroupedArgs& a, bool trace, hipStream_t s, const 
     // k_router_exact takes (777 tokens x 128 experts: 27 us there)
     if (et * rt <= 256) launch(k_router_exact_small, dim3(et, rt), dim3(64 * (1 + kPcProducers)), 0, s, a);
     else launch(k_router_exact, dim3((a.ne + 7) / 8, (nt + 7) / 8), dim3(64), 0, s, a);
-    launch(k_select_batch, dim3(nt), dim3(64), select_lds_bytes(a.ne, a.d, kExactGroupWide), s, a);
-    launch(k_group_scan, dim3(1), dim3(1024), 0, s, a);
+    if (nt <= kSelMax) {
+        launch(k_select_group, dim3(1), dim3(1024), 0, s, a);
+    } else {
+        launch(k_select_batch, dim3((nt + 3) / 4), dim3(256), 0, s, a);
+        launch(k_group_scan, dim3(1), dim3(1024), 0, s, a);
+    }
     if (a.kq) {
         if (launch_kq_gemms(a, trace, s, ev)) return -19;
         launch(k_combine_batch, dim3((unsigned)std::min<size_t>(((size_t)nt * (a.d / 4) + 255) / 256, 2048)), dim3(256), 0, s, a);

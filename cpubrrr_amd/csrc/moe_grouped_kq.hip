@@ -89,7 +89,6 @@ __global__ __launch_bounds__(256) void k_prep_batch_kq(GroupedArgs a) {
     float* xnl = xs + d;
     float* scratch = xnl + d;
     norm_into(a.x + (size_t)t * d, a.norm_w, d, a.eps, a.norm, a.norm_nt, a.apply_norm, xs, xnl, scratch);
-    if (tid == 0) a.inv[t] = a.apply_norm ? scratch[16] : 1.0f;
     // 8 consecutive elements per thread, 32 threads per superblock
     for (int e0 = tid * 8; e0 < d; e0 += 256 * 8) {
         float v[8];

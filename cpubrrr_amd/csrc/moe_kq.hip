@@ -71,7 +71,7 @@ __global__ __launch_bounds__(1024) void k_gateup_kq(KqArgs a) {
         if (ranked) select_rank_wg(a.sel, smem, blockIdx.x == 0 ? a.sel.logits : nullptr, pre);
         // ids only; workgroup 0 publishes the softmax weights once its
         // weight loads are in flight
-        if (q == 0) select_topk_wave(a.sel, smem, &ssel, false, nullptr, ranked, true);
+        if (q == 0) select_topk_wave(a.sel, smem, &ssel, nullptr, ranked, true);
         __syncthreads();
         e = uniform(ssel.ids[ei]);
     } else {

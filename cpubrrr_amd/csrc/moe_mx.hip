@@ -85,7 +85,7 @@ __global__ __launch_bounds__(128 * kMaxParts) __attribute__((amdgpu_waves_per_eu
         // ids only; workgroup 0 publishes the softmax weights once its weight
         // loads are in flight
         if (w == 0)
-            select_topk_wave(a.sel, smem, &ssel, false, &pre,
+            select_topk_wave(a.sel, smem, &ssel, &pre,
                              false, true);
         // barrier on LDS only (s_barrier without a wait for the activation loads)
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");

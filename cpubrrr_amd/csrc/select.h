@@ -15,11 +15,9 @@
 
 namespace cpb {
 
-// candidates whose exact serial logits are computed side by side: four in
-// the decode kernels (their LDS budget), eight in the batched selection
+// candidates whose exact serial logits are computed side by side (the decode
+// kernels' LDS budget)
 constexpr int kExactGroup = 4;
-constexpr int kExactGroupWide = 8;
-CPB_DEV_HOST_INLINE constexpr int exact_group(int cand) { return cand > 1 ? kExactGroupWide : kExactGroup; }
 // LDS floats per candidate's product row: d plus the chain's look-ahead slack
 // (64 floats), a multiple of 4 (16-byte reads) that spreads the chain lanes
 // over the banks
@@ -49,13 +47,12 @@ struct Selection {
 // reaches the lowest lower bound of the provisional top-k, then rank those
 // exactly (descending, lowest index first).  sL / sH: LDS values and upper
 // bounds of all NE experts; sSel: LDS [K] provisional choice, overwritten;
-// pst: LDS scratch of exact_group(CAND) * exact_stride(d) floats, then NE
-// ints.  One wavefront.
-template <int CAND, int CHUNK>
+// pst: LDS scratch of kExactGroup * exact_stride(d) floats, then NE ints.
+// One wavefront.
 CPB_DEV void exact_reselect(double* sL, const double* sH, int* sSel, int NE, int K, const float* __restrict__ router_w,
                             const float* __restrict__ router_b, const float* __restrict__ xn, int d, float* pst) {
     const int lane = threadIdx.x & 63;
-    constexpr int NG = exact_group(CAND);
+    constexpr int NG = kExactGroup;
     int* sList = (int*)(pst + NG * exact_stride(d));   // [NE] every candidate, ascending
     // candidates: intervals reaching the lowest lower bound of the selected
     double tau = 1e300;
@@ -87,60 +84,19 @@ CPB_DEV void exact_reselect(double* sL, const double* sH, int* sSel, int NE, int
         // the group's candidates
         const int ng = min(NG, nl - g0);
         const int* sCand = sList + g0;
-        if constexpr (CAND == 1) {
-            // one 16-byte load pair per lane in flight (few registers)
-            for (int c = 0; c < ng; c++) {
-                const int ec = sCand[c];
-                const __amdgpu_buffer_rsrc_t rw = buf_rsrc(router_w + (size_t)ec * d, (uint32_t)d * 4);
-                for (int j = 4 * lane; j < d; j += 256) {
-                    const u32x4 w4 = __builtin_amdgcn_raw_buffer_load_b128(rw, (uint32_t)j * 4, 0, 0);
-                    const u32x4 x4 = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)j * 4, 0, 0);
-                    float4 p4;
-                    p4.x = __fmul_rn(__uint_as_float(w4[0]), __uint_as_float(x4[0]));
-                    p4.y = __fmul_rn(__uint_as_float(w4[1]), __uint_as_float(x4[1]));
-                    p4.z = __fmul_rn(__uint_as_float(w4[2]), __uint_as_float(x4[2]));
-                    p4.w = __fmul_rn(__uint_as_float(w4[3]), __uint_as_float(x4[3]));
-                    *(float4*)(pst + c * stride + j) = p4;
-                }
-            }
-        } else {
-            // CAND candidates' rows (CHUNK 16-byte loads per lane each) in flight per round
-            for (int c0 = 0; c0 < ng; c0 += CAND) {
-                for (int j0 = 0; j0 < d; j0 += 256 * CHUNK) {
-                    u32x4 x4[CHUNK], w4[CAND][CHUNK];
-    #pragma unroll
-                    for (int k = 0; k < CHUNK; k++) {
-                        const int j = j0 + 256 * k + 4 * lane;
-                        x4[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, j < d ? (uint32_t)j * 4 : kOffNone, 0, 0);
-                    }
-    #pragma unroll
-                    for (int ci = 0; ci < CAND; ci++) {
-                        const int c = c0 + ci;
-                        const int ec = sCand[c < ng ? c : 0];
-                        const __amdgpu_buffer_rsrc_t rw = buf_rsrc(router_w + (size_t)ec * d, c < ng ? (uint32_t)d * 4 : 0u);
-    #pragma unroll
-                        for (int k = 0; k < CHUNK; k++) {
-                            const int j = j0 + 256 * k + 4 * lane;
-                            w4[ci][k] = __builtin_amdgcn_raw_buffer_load_b128(rw, j < d ? (uint32_t)j * 4 : kOffNone, 0, 0);
-                        }
-                    }
-    #pragma unroll
-                    for (int ci = 0; ci < CAND; ci++) {
-                        const int c = c0 + ci;
-    #pragma unroll
-                        for (int k = 0; k < CHUNK; k++) {
-                            const int j = j0 + 256 * k + 4 * lane;
-                            if (c < ng && j < d) {
-                                float4 p4;
-                                p4.x = __fmul_rn(__uint_as_float(w4[ci][k][0]), __uint_as_float(x4[k][0]));
-                                p4.y = __fmul_rn(__uint_as_float(w4[ci][k][1]), __uint_as_float(x4[k][1]));
-                                p4.z = __fmul_rn(__uint_as_float(w4[ci][k][2]), __uint_as_float(x4[k][2]));
-                                p4.w = __fmul_rn(__uint_as_float(w4[ci][k][3]), __uint_as_float(x4[k][3]));
-                                *(float4*)(pst + c * stride + j) = p4;
-                            }
-                        }
-                    }
-                }
+        // one 16-byte load pair per lane in flight (few registers)
+        for (int c = 0; c < ng; c++) {
+            const int ec = sCand[c];
+            const __amdgpu_buffer_rsrc_t rw = buf_rsrc(router_w + (size_t)ec * d, (uint32_t)d * 4);
+            for (int j = 4 * lane; j < d; j += 256) {
+                const u32x4 w4 = __builtin_amdgcn_raw_buffer_load_b128(rw, (uint32_t)j * 4, 0, 0);
+                const u32x4 x4 = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)j * 4, 0, 0);
+                float4 p4;
+                p4.x = __fmul_rn(__uint_as_float(w4[0]), __uint_as_float(x4[0]));
+                p4.y = __fmul_rn(__uint_as_float(w4[1]), __uint_as_float(x4[1]));
+                p4.z = __fmul_rn(__uint_as_float(w4[2]), __uint_as_float(x4[2]));
+                p4.w = __fmul_rn(__uint_as_float(w4[3]), __uint_as_float(x4[3]));
+                *(float4*)(pst + c * stride + j) = p4;
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -151,35 +107,11 @@ CPB_DEV void exact_reselect(double* sL, const double* sH, int* sSel, int NE, int
             const float* pr = pst + lane * stride;
             float acc = router_b ? router_b[e] : 0.0f;
             int j = 0;
-            if constexpr (CAND > 1) {
-                // full groups of 32 products streamed from LDS (the next
-                // group's reads issued before the current group's adds; the
-                // look-ahead reads at most 64 floats past d, inside the
-                // stride's slack).  64 registers: the wide variant only.
-                const int nfull = d / 32;
-                uint32_t ra = lds_addr(pr);
-                f32x4 ga[8], gb[8];
-                lds_read8(ga, ra);
-                for (int m = 0;; m += 2) {
-                    lds_read8(gb, ra + 128);
-                    lds_wait_older8(ga);
-                    if (m >= nfull) break;
-                    acc = serial_add32(ga, acc);
-                    lds_read8(ga, ra + 256);
-                    lds_wait_older8(gb);
-                    if (m + 1 >= nfull) break;
-                    acc = serial_add32(gb, acc);
-                    ra += 256;
-                }
-                lds_wait_all();
-                j = nfull * 32;
-            } else {
-                for (; j + 32 <= d; j += 32) {
-                    f32x4 v[8];
+            for (; j + 32 <= d; j += 32) {
+                f32x4 v[8];
 #pragma unroll
-                    for (int u = 0; u < 8; u++) v[u] = *(const f32x4*)(pr + j + 4 * u);
-                    acc = serial_add32(v, acc);
-                }
+                for (int u = 0; u < 8; u++) v[u] = *(const f32x4*)(pr + j + 4 * u);
+                acc = serial_add32(v, acc);
             }
             for (; j < d; j++) acc = __fadd_rn(acc, pr[j]);
             sL[e] = (double)acc;
@@ -222,8 +154,8 @@ struct SelectIn {
     int32_t* fallback;       // [1]
 };
 // LDS bytes select_topk_wave may use (its exact fallback)
-CPB_DEV_HOST_INLINE size_t select_lds_bytes(int ne, int d, int group = kExactGroup) {
-    return sizeof(double) * 2 * ne + 64 + sizeof(float) * group * exact_stride(d) + sizeof(int) * ne;
+CPB_DEV_HOST_INLINE size_t select_lds_bytes(int ne, int d) {
+    return sizeof(double) * 2 * ne + 64 + sizeof(float) * kExactGroup * exact_stride(d) + sizeof(int) * ne;
 }
 
 // Wave-wide maximum of a 32-bit unsigned value via DPP (quad swaps, half-row
@@ -261,14 +193,13 @@ CPB_DEV float f32_down(double x) {
 // Rare path of select_topk_wave (pointer and scalar
 // arguments only, so the caller needs no stack): exact_reselect over the LDS
 // image the caller wrote.
-template <int CAND, int CHUNK>
-CPB_DEV void select_exact_path(unsigned char* lds, int NE, int K, const float* router_w,
-                                                            const float* router_b, const float* xn, int d) {
+CPB_DEV void select_exact_path(unsigned char* lds, int NE, int K, const float* router_w, const float* router_b,
+                               const float* xn, int d) {
     double* sL = (double*)lds;
     double* sH = sL + NE;
     int* sSel = (int*)(sH + NE);
     float* xst = (float*)(lds + sizeof(double) * 2 * NE + 64);
-    exact_reselect<CAND, CHUNK>(sL, sH, sSel, NE, K, router_w, router_b, xn, d, xst);
+    exact_reselect(sL, sH, sSel, NE, K, router_w, router_b, xn, d, xst);
 }
 
 // One wavefront's LDS writes visible to its later LDS reads (a wave's LDS
@@ -365,9 +296,6 @@ CPB_DEV void select_rank_wg(const SelectIn& s, unsigned char* lds, float* logits
     __syncthreads();
 }
 
-// EXACT_CAND / EXACT_CHUNK: router rows (and 16-byte loads per lane of each)
-// in flight on the exact path; EXACT_CAND > 1 also streams the serial chains'
-// LDS reads ahead (registers: the decode kernels keep both small)
 // ranked: select_rank_wg ran first (the logits were published there); the
 // wave certifies its LDS ranking and, on the rare exact path, reloads the
 // intervals.
@@ -376,10 +304,8 @@ CPB_DEV void select_rank_wg(const SelectIn& s, unsigned char* lds, float* logits
 // published ids / weights follow from select_publish, which workgroup 0 runs
 // once its loads are in flight.
 CPB_DEV void select_publish(const SelectIn& s, const Selection* out);
-template <int EXACT_CAND = 1, int EXACT_CHUNK = 1>
-CPB_DEV void select_topk_wave(const SelectIn& s, unsigned char* lds, Selection* out, bool publish_logits = false,
-                              const SelectPre* pre = nullptr, bool ranked = false,
-                              bool defer = false) {
+CPB_DEV void select_topk_wave(const SelectIn& s, unsigned char* lds, Selection* out, const SelectPre* pre = nullptr,
+                              bool ranked = false, bool defer = false) {
     const int lane = threadIdx.x & 63;
     const int NE = s.ne, K = s.k;
     double lv[4] = {0.0, 0.0, 0.0, 0.0}, bv[4] = {0.0, 0.0, 0.0, 0.0};
@@ -515,7 +441,7 @@ CPB_DEV void select_topk_wave(const SelectIn& s, unsigned char* lds, Selection* 
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        select_exact_path<EXACT_CAND, EXACT_CHUNK>(lds, NE, K, s.router_w, s.router_b, s.xn, s.d);
+        select_exact_path(lds, NE, K, s.router_w, s.router_b, s.xn, s.d);
         if (lane < K) { my_e = sSel[lane]; my_l = (float)sL[my_e]; }
     }
     if (defer) {
@@ -547,16 +473,8 @@ CPB_DEV void select_topk_wave(const SelectIn& s, unsigned char* lds, Selection* 
     }
     if (lane == 0) out->fallback = bad ? 1 : 0;
     // trace outputs and the routed ids / weights for later launches (by one
-    // workgroup, or by this one when it alone selects for its token)
-    if (publish_logits) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int e = lane + 64 * j;
-            if (e < NE) s.logits[e] = lf[j];
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane < K) s.logits[my_e] = my_l;
-    } else if (blockIdx.x == 0 && blockIdx.y == 0) {
+    // workgroup)
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
         if (!ranked) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {

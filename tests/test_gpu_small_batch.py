@@ -55,3 +55,15 @@ def test_kq_small_batches(gpu, d, dff, ne, k, n_tok, down, same):
     L = synth.qwen_layer(d, dff, ne, k, seed=22, down_type=down)
     X = np.stack([synth.token(d, 22, 0 if same else i) for i in range(n_tok)])
     check(L, MoeConfig.qwen3(d=d, n_expert=ne, top_k=k, d_ff=dff, max_tokens=n_tok, down_type=down), X, "qwen")
+
+
+@pytest.mark.parametrize("ne,k,n_tok", [(32, 4, 5), (128, 8, 64), (128, 8, 65)])    # one launch up to 64 tokens, two beyond
+def test_batched_selection_ties(gpu, ne, k, n_tok):
+    """Equal logits (equal router rows): the lowest index wins, as in the reference."""
+    print(f"case batched selection ties ne={ne} k={k} n_tok={n_tok}", flush=True)
+    L = synth.gptoss_layer(384, 64, ne, k, seed=23)
+    W = L["router_w"].reshape(ne, 384)
+    W[: ne // 2] = W[ne // 2:]                       # every logit twice
+    W[1] = W[2] = W[0]                               # and one four times
+    X = np.stack([synth.token(384, 23, i) for i in range(n_tok)])
+    check(L, MoeConfig.gptoss(d=384, n_expert=ne, top_k=k, d_ff=64, max_tokens=n_tok), X, "gptoss")
