@@ -255,11 +255,14 @@ __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(
         const uint32_t xo = tx < nt ? (uint32_t)tx * d * 4 + u0 * 64 + (4 * r + (i & 3)) * 4 : kOffNone;
         f32x4 wv[kPcAhead][UP];
         float xv[kPcAhead][UP];
+        // (the whole offset in the vector offset: the scalar one is not part
+        // of the buffer's range check)
         auto load = [&](int s, int ch) {
+            const uint32_t wc = wo + (uint32_t)ch * (kPcChunk * 64), xc = xo + (uint32_t)ch * (kPcChunk * 4);
 #pragma unroll
             for (int u = 0; u < UP; u++) {
-                wv[s][u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo + u * 1024, (uint32_t)ch * (kPcChunk * 64), 0));
-                xv[s][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, xo + u * 64, (uint32_t)ch * (kPcChunk * 4), 0));
+                wv[s][u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wc + u * 1024, 0, 0));
+                xv[s][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, xc + u * 64, 0, 0));
             }
             __builtin_amdgcn_sched_barrier(0);    // one order of requests everywhere: exact waits
         };
