@@ -530,30 +530,39 @@ CPB_DEV v16f mx_block_mfma_b(const u32x4& w, const u32x4& x0, const u32x4& x1, u
     }
 }
 
-// LDS staging of one k-part's activations for a 32-token tile: per block i
-// and token ti a 64-byte slot whose four 16-byte chunks are XOR-swizzled by
-// the token (chunk c at position c ^ swz(ti)), then room for 512 scales (15 x
-// 32 used).  The swizzle puts the reads (lane ti reads chunk 2hb or 2hb + 1 of
-// slot ti) on distinct banks in every group of 8 and of 16 lanes (80-byte
-// padded slots had 2.75 M conflict cycles per gate/up launch).
+// A k-part's two chains (blocks 0-7 and 8-14) are staged and multiplied as two
+// sub-parts.  LDS staging of one sub-part's activations for a 32-token tile:
+// per block i < 8 and token ti a 64-byte slot whose four 16-byte chunks are
+// XOR-swizzled by the token (chunk c at position c ^ swz(ti)), then the 8 x 32
+// scales; the staging's last rounds fill up to whole rounds of NW waves.  The
+// swizzle puts the reads (lane ti reads chunk 2hb or 2hb + 1 of slot ti) on
+// distinct banks in every group of 8 and of 16 lanes (80-byte padded slots had
+// 2.75 M conflict cycles per gate/up launch).
 constexpr int kSlot = 64;
-constexpr int kStageBlk = 15;
-constexpr int kStageBytes = kStageBlk * 32 * kSlot + 512 * 4;
+constexpr int kSub = kSubUnits;               // blocks of a sub-part (the second has 7)
+static_assert(kSub == 8 && kBlkPerPart == 15, "sub-parts of 8 and 7 blocks");
 CPB_DEV_HOST_INLINE int stage_swz(int ti) { return ((ti >> 1) ^ (ti >> 2)) & 3; }
+// image loads of 1 KB (half a block's tokens) and scale loads of 64 per wave and sub-part
+constexpr int stage_img(int nw) { return (2 * kSub + nw - 1) / nw; }
+constexpr int stage_sc(int nw) { return (kSub / 2 + nw - 1) / nw; }
+constexpr int stage_bytes(int nw) { return nw * (stage_img(nw) * 1024 + stage_sc(nw) * 256); }
+// Waves per workgroup, each with two 32-row tiles
+constexpr int kGemmWaves = 4;
 
-// Workgroup sizes of the grouped GEMMs.  Gate/up: 4 waves, so that two
-// workgroups share a CU (LDS 2 x 65 KB, <= 256 registers per lane) and one's
-// barriers, prologue and SwiGLU epilogue overlap the other's k-part loop.
-// Down (a short epilogue): 8 waves, whose row tiles share one staged
-// activation tile.
-constexpr int kGuThreads = 256, kDnThreads = 512;
+// The two staging buffers (a k-part's first and second sub-part): separate
+// objects, so that the compiler can tell the buffer being filled from the one
+// being read (it would otherwise wait for every direct load before each read)
+constexpr int kStageBytes = stage_bytes(kGemmWaves);
+__shared__ __align__(16) unsigned char g_stage0[kStageBytes];
+__shared__ __align__(16) unsigned char g_stage1[kStageBytes];
 
-
-// Direct global-to-LDS staging of k-part q (no staging registers): each
-// wavefront instruction writes 1 KB of LDS, lane L at byte 16 L, so lane L
-// fetches the chunk the swizzled layout puts there (token h*16 + L/4 of the
-// block, chunk (L & 3) ^ swz(token)); the scales take 8 instructions of 64
-// (the last half past block 14 reads nothing).
+// Direct global-to-LDS staging (no staging registers): each wavefront
+// instruction writes 1 KB of LDS, lane L at byte 16 L, so lane L fetches the
+// chunk the swizzled layout puts there (token h*16 + L/4 of the block, chunk
+// (L & 3) ^ swz(token)); the scales take 64 per instruction.
+// An offset beyond both buffers (at most 16384 rows x 120 blocks x 64 bytes),
+// twice of which is beyond them too:
+constexpr uint32_t kStageNone = 0x40000000u;
 struct DmaPlan {
     __amdgpu_buffer_rsrc_t ri, rs;
     uint32_t vbase0, vbase1, sbase;  // bytes: block 0 of the lane's chunk in token half 0 / 1, its scale
@@ -564,333 +573,377 @@ CPB_DEV DmaPlan dma_plan(const uint8_t* img, const float* sc, size_t rows, int n
     p.ri = buf_rsrc(img, (uint32_t)(rows * nbk * kImg));
     p.rs = buf_rsrc(sc, (uint32_t)(rows * nbk * 4));
     const int t0 = L >> 2, t1 = 16 + (L >> 2), r0 = src[t0], r1 = src[t1];
-    p.vbase0 = r0 >= 0 ? (uint32_t)r0 * nbk * kImg + (uint32_t)(((L & 3) ^ stage_swz(t0)) << 4) : kOffNone;
-    p.vbase1 = r1 >= 0 ? (uint32_t)r1 * nbk * kImg + (uint32_t)(((L & 3) ^ stage_swz(t1)) << 4) : kOffNone;
+    p.vbase0 = r0 >= 0 ? (uint32_t)r0 * nbk * kImg + (uint32_t)(((L & 3) ^ stage_swz(t0)) << 4) : kStageNone;
+    p.vbase1 = r1 >= 0 ? (uint32_t)r1 * nbk * kImg + (uint32_t)(((L & 3) ^ stage_swz(t1)) << 4) : kStageNone;
     const int rs_ = src[L & 31];
-    p.sbase = rs_ >= 0 ? (uint32_t)rs_ * nbk * 4 : kOffNone;
+    p.sbase = rs_ >= 0 ? (uint32_t)rs_ * nbk * 4 : kStageNone;
     return p;
 }
-template <int NT>
-CPB_DEV void stage_dma(const DmaPlan& p, int nbk, int q, unsigned char* st) {
+// Sub-part sp (k-part sp / 2, its blocks 0-7 or 8-14) into st.  Every wave
+// issues the same number of loads whatever the sub-part: the pieces past its
+// last block, past the last k-part and past the last round read nothing and
+// write zeros.  So a wave's loads are counted exactly, and the wait for these
+// does not wait for what is requested after them.
+template <int NW>
+CPB_DEV void stage_dma(const DmaPlan& p, int nbk, int sp, unsigned char* st) {
     // the wave index as a scalar: every condition and LDS address below is
     // then scalar work
     const int w = uniform((int)(threadIdx.x >> 6)), L = threadIdx.x & 63;
-    const int lim = min(kBlkPerPart, nbk - q * kBlkPerPart);
+    const int b0 = (sp >> 1) * kBlkPerPart + (sp & 1) * kSub;
+    const int lim = min(kSub - (sp & 1), nbk - b0);
 #pragma unroll
-    for (int k = 0; k < (2 * kBlkPerPart + NT / 64 - 1) / (NT / 64); k++) {
-        const int m = w + k * (NT / 64), i = m >> 1, h = m & 1;
-        if (m < 2 * kBlkPerPart) {
-            const uint32_t off = i < lim ? (h ? p.vbase1 : p.vbase0) + (uint32_t)(q * kBlkPerPart + i) * kImg : kOffNone;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(p.ri, (lds_void_g*)(st + (i * 32 + h * 16) * kSlot), 16, off, 0, 0, 0);
-        }
+    for (int k = 0; k < stage_img(NW); k++) {
+        const int m = w + k * NW, i = m >> 1, h = m & 1;
+        const uint32_t add = (uint32_t)(b0 + i) * kImg + (i < lim ? 0u : kStageNone);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(p.ri, (lds_void_g*)(st + m * 1024), 16, (h ? p.vbase1 : p.vbase0) + add, 0, 0, 0);
     }
 #pragma unroll
-    for (int k = 0; k < (8 + NT / 64 - 1) / (NT / 64); k++) {
-        const int n = w + k * (NT / 64), i = 2 * n + (L >> 5);
-        if (n < 8) {
-            const uint32_t off = i < lim ? p.sbase + (uint32_t)(q * kBlkPerPart + i) * 4 : kOffNone;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(p.rs, (lds_void_g*)(st + kStageBlk * 32 * kSlot + n * 256), 4, off, 0, 0, 0);
-        }
+    for (int k = 0; k < stage_sc(NW); k++) {
+        const int n = w + k * NW, i = 2 * n + (L >> 5);
+        const uint32_t off = p.sbase + (uint32_t)(b0 + i) * 4 + (i < lim ? 0u : kStageNone);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(p.rs, (lds_void_g*)(st + NW * stage_img(NW) * 1024 + n * 256), 4, off, 0, 0, 0);
     }
 }
-// the two staging buffers of the DMA-staged GEMMs, as separate objects so
-// that the compiler can tell the buffer being filled from the one being read
-__shared__ __align__(16) unsigned char g_stage0[kStageBytes];
-__shared__ __align__(16) unsigned char g_stage1[kStageBytes];
 
-// Weight operand of one k-part for the lane's row: unit u (0 = the e8m0
-// bytes, 1..15 = blocks) sits at byte off + u * ustride of the expert's
-// stream; rs covers the expert's whole stream (out-of-range offsets read 0).
+// Weight operands of the lane's two rows (one in each of the wave's two row
+// tiles): a row's units (16 per k-part: the e8m0 bytes, then 15 blocks) follow
+// each other at ustride bytes from off in the expert's stream; rs covers the
+// expert's whole stream (out-of-range offsets read 0).
 struct WeightStream {
     __amdgpu_buffer_rsrc_t rs;
-    uint32_t off, ustride, pstride;      // bytes: lane's unit 0 of k-part 0, unit step, k-part step
+    uint32_t off[2], ustride;
 };
-CPB_DEV u32x4 wload(const WeightStream& ws, int q, int u) {
-    return __builtin_amdgcn_raw_buffer_load_b128(ws.rs, ws.off + (uint32_t)q * ws.pstride + (uint32_t)u * ws.ustride, 0, 0);
+// Both K halves of the instruction's A operand (both lane halves) take the same
+// 16 bytes of a row.  So that no byte is loaded twice, one load brings two
+// units, lanes 0-31 unit 2 j + 1 and lanes 32-63 unit 2 j + 2 (a k-part's last
+// pair: block 14 and the next k-part's e8m0 bytes), and each goes to both
+// halves by v_permlane32_swap, which works in place: the pair's registers hold
+// y until the odd block has used it.  Half the L1 traffic and half the
+// registers of a load per unit.
+CPB_DEV void split_pair(const u32x4& v, u32x4& x, u32x4& y) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v[c], v[c], false, false);
+        x[c] = r[0];
+        y[c] = r[1];
+    }
 }
 
-// The k-part loop shared by the two grouped GEMMs.  Per k-part, D = A(rows)
-// x B(tokens) per block on the matrix cores and acc = fma(D, xsb, acc) in
-// block order, in two chains (blocks 0-7 and 8-14, as the decode kernels'
-// two wavefronts per k-part), the chains added to the total in order.
+// A 16-pass MFMA's results may be read 19 wait states after it.  Where only the
+// other tile's sixteen fmas, one MFMA and waits lie between, the compiler left
+// 17 (the last blocks' sums were read too early, wrong on every run): mfma_gap
+// adds 8 there.  Elsewhere at least three LDS reads lie between as well.
+CPB_DEV void mfma_gap() { asm volatile("s_nop 7"); }
+
+// The loop shared by the two grouped GEMMs: two row tiles x one token tile per
+// wave, whose activations both tiles' products read from LDS once (a b128 read
+// takes the LDS 16 cycles, so at one tile per read the four SIMDs' reads took
+// 61 ns per block and tile against 28 of matrix-core and 27 of VALU work: two,
+// three and four waves per SIMD all ran at that rate).  Per
+// block, D = A(rows) x B(tokens) on the matrix cores and acc = fma(D, xsb, acc)
+// in block order, in two chains per k-part (its sub-parts, as the decode
+// kernels' two wavefronts per k-part), the chains added to the total in order.
 //
-// Software pipeline: block i + 1's MFMA is issued before block i's sixteen
-// fmas (two D register sets), so the matrix core and the VALU run side by
-// side; each weight register is refilled with the next k-part's unit right
-// after its MFMA has been issued (one k-part of lead time, 16 units of
-// registers instead of 32).  Two LDS staging buffers alternate for the
-// activations: right after the barrier that opens k-part q, the direct loads
-// of k-part q + 1 go into the other buffer (every wave has finished reading it
-// in k-part q - 1), so one barrier per k-part suffices; the barrier's release
-// fence makes each wave wait for its own direct loads first.
-// TRACE writes the int32 block sums S = D * 2^(128 - e) of valid rows.
-template <bool TRACE, int NT>
-CPB_DEV v16f grouped_parts(const WeightStream& ws, int P, const uint8_t* img, const float* sc,
-                           size_t rows, int nbk, const int* src, int lane, int32_t* tb, bool trace_ok,
-                           float* bias_lds, float bias_v, int nbias) {
+// Software pipeline: the two tiles' MFMAs and the other tile's sixteen fmas
+// alternate, so the matrix core and the VALU run side by side; each weight pair
+// is requested again, a k-part ahead, right after it has been taken apart.  Two
+// LDS buffers alternate: right after the barrier that opens a sub-part the
+// direct loads of the next go into the buffer that every wave has finished
+// reading.  Before that barrier a wave waits for its own direct loads and not
+// for the weight pairs requested since (a full fence there, which drained
+// them, exposed a memory latency per k-part).
+// TRACE writes the int32 block sums S = D * 2^(128 - e) of valid rows (tb, per
+// row tile; null: none).
+constexpr uint32_t s_waitcnt_vm(int n) { return (uint32_t)((n & 15) | 0x70 | 0xF00 | ((n >> 4) << 14)); }   // vmcnt(n) only
+template <bool TRACE, int NW>
+CPB_DEV void grouped_parts(const WeightStream& ws, int P, const uint8_t* img, const float* sc, size_t rows, int nbk,
+                           const int* src, int lane, int32_t* const (&tb)[2], v16f (&tot)[2]) {
     const int ti = lane & 31, hb = lane >> 5;
     // the lane's two 16-byte chunks (2hb, 2hb + 1) of its token's slot
-    const int o0 = ((2 * hb) ^ stage_swz(ti)) << 4, o1 = ((2 * hb + 1) ^ stage_swz(ti)) << 4;
-    u32x4 wv[kUnits];
-#pragma unroll
-    for (int u = 0; u < kUnits; u++) wv[u] = wload(ws, 0, u);
+    const int o0 = ti * kSlot + (((2 * hb) ^ stage_swz(ti)) << 4), o1 = ti * kSlot + (((2 * hb + 1) ^ stage_swz(ti)) << 4);
+    const int os = NW * stage_img(NW) * 1024 + ti * 4;
     const DmaPlan dp = dma_plan(img, sc, rows, nbk, src);
-    stage_dma<NT>(dp, nbk, 0, g_stage0);
-    v16f tot = {};
-    // k-part q on the activations staged in st; the next k-part's go to nx
-    auto kpart = [&](int q, unsigned char* st, unsigned char* nx) {
-        __syncthreads();                     // k-part q's activations have landed
-        // past the last k-part the refills read out of range (zeros, no traffic)
-        const int qn = q + 1 < P ? q + 1 : 0x7fff;
-        const u32x4 ex = wv[0];
-        wv[0] = wload(ws, qn, 0);
-        if (q + 1 < P) stage_dma<NT>(dp, nbk, q + 1, nx);
-        const unsigned char* xp = st + ti * kSlot;
-        const float* sl = (const float*)(st + kStageBlk * 32 * kSlot) + ti;
-        v16f acc = {}, Dc, Dn;
-        float sc_c, sc_n;
-        // activation operands two blocks ahead: buffer j & 1 holds block j's
-        // until its MFMA is issued, then takes block j + 2's
-        u32x4 xa[2][2];
-        float sa[2];
+    auto wload = [&](int m, uint32_t unit) {
+        return __builtin_amdgcn_raw_buffer_load_b128(ws.rs, ws.off[m] + unit * ws.ustride, 0, 0);
+    };
+    u32x4 ex[2], wp[2][8];
+    ex[0] = wload(0, 0);
+    ex[1] = wload(1, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    stage_dma<NW>(dp, nbk, 0, g_stage0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            xa[j][0] = *(const u32x4*)(xp + j * 32 * kSlot + o0);
-            xa[j][1] = *(const u32x4*)(xp + j * 32 * kSlot + o1);
-            sa[j] = sl[j * 32];
-        }
-        {
-            sc_c = sa[0];
-            Dc = mx_block_mfma<0>(wv[1], xa[0][0], xa[0][1], ex[0]);
-            wv[1] = wload(ws, qn, 1);
-            xa[0][0] = *(const u32x4*)(xp + 2 * 32 * kSlot + o0);
-            xa[0][1] = *(const u32x4*)(xp + 2 * 32 * kSlot + o1);
-            sa[0] = sl[2 * 32];
-        }
+    for (int j = 0; j < 8; j++) {
+        wp[0][j] = wload(0, 2 * j + 1 + hb);
+        wp[1][j] = wload(1, 2 * j + 1 + hb);
+        __builtin_amdgcn_sched_barrier(0);   // in the loop's order: exact waits there
+    }
+    tot[0] = tot[1] = v16f{};
+    for (int q = 0; q < P; q++) {
 #pragma unroll
-        for (int i = 0; i < kBlkPerPart; i++) {
-            if (i + 1 < kBlkPerPart) {
-                const int j = i + 1, bj = j & 1;
-                sc_n = sa[bj];
-                Dn = mx_block_mfma_b(wv[1 + j], xa[bj][0], xa[bj][1], ex[j >> 2], j);
-                wv[1 + j] = wload(ws, qn, 1 + j);
-                if (j + 2 < kBlkPerPart) {
-                    xa[bj][0] = *(const u32x4*)(xp + (j + 2) * 32 * kSlot + o0);
-                    xa[bj][1] = *(const u32x4*)(xp + (j + 2) * 32 * kSlot + o1);
-                    sa[bj] = sl[(j + 2) * 32];
-                }
-            }
-            // keep the order as written (the scheduler would sink the reads
-            // next to their MFMA)
+        for (int half = 0; half < 2; half++) {
+            const int sp = 2 * q + half, nblk = kSub - half;
+            // the sub-part's activations have landed: the wave's own (all but
+            // the 2 x 4 weight pairs requested since), then every wave's
+            asm volatile("" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
-            if (TRACE) {
-                const int b = q * kBlkPerPart + i;
-                const uint32_t eb = (ex[i >> 2] >> (8 * (i & 3))) & 0xffu;
+            __builtin_amdgcn_s_waitcnt(s_waitcnt_vm(8));
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
+            const unsigned char* st = half ? g_stage1 : g_stage0;
+            stage_dma<NW>(dp, nbk, sp + 1, half ? g_stage0 : g_stage1);
+            __builtin_amdgcn_sched_barrier(0);
+            const unsigned char* x0 = st + o0;
+            const unsigned char* x1 = st + o1;
+            const unsigned char* sl = st + os;
+            v16f acc[2] = {}, D[2];
+            u32x4 xa[2][2], X[2], Y[2];
+            float sa[2], sd = 0.0f;
+            auto xread = [&](int j) {
+                xa[j & 1][0] = *(const u32x4*)(x0 + j * 32 * kSlot);
+                xa[j & 1][1] = *(const u32x4*)(x1 + j * 32 * kSlot);
+                sa[j & 1] = *(const float*)(sl + j * 128);
+            };
+            auto trace = [&](int m, int i) {
+                const int bl = half * kSub + i, b = q * kBlkPerPart + bl;
+                const uint32_t eb = (ex[m][bl >> 2] >> (8 * (bl & 3))) & 0xffu;
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int rl = 8 * (r >> 2) + 4 * hb + (r & 3);
                     const int e_r = __shfl((int)eb, rl);
-                    if (trace_ok && b < nbk) tb[rl * (size_t)nbk + b] = (int)ldexpf(Dc[r], 128 - e_r);
+                    if (tb[m] && b < nbk) tb[m][rl * (size_t)nbk + b] = (int)ldexpf(D[m][r], 128 - e_r);
+                }
+            };
+            auto add = [&](int m, int i, float s) {
+                if (TRACE) trace(m, i);
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[m][r] = fmaf(D[m][r], s, acc[m][r]);
+            };
+            // block i of tile m: an even block's pair is taken apart first (in
+            // place), and requested again once the odd one has used its half
+            auto refill = [&](int m, int i) { wp[m][half * 4 + (i >> 1)] = wload(m, 16 * (q + 1) + half * 8 + (i & ~1) + 1 + hb); };
+            auto mul = [&](int m, int i) {
+                const int bl = half * kSub + i;
+                if (!(i & 1)) split_pair(wp[m][half * 4 + (i >> 1)], X[m], Y[m]);
+                D[m] = mx_block_mfma_b(i & 1 ? Y[m] : X[m], xa[i & 1][0], xa[i & 1][1], ex[m][bl >> 2], bl);
+                if (i & 1) refill(m, i);
+            };
+            xread(0);
+            xread(1);
+#pragma unroll
+            for (int i = 0; i < nblk; i++) {
+                mul(0, i);
+                // keep the order as written
+                __builtin_amdgcn_sched_barrier(0);
+                if (i) {
+                    if (i + 1 >= nblk) mfma_gap();
+                    add(1, i - 1, sd);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                mul(1, i);
+                sd = sa[i & 1];
+                if (i + 2 < nblk) xread(i + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                if (i + 2 >= nblk) mfma_gap();
+                add(0, i, sd);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            mfma_gap();
+            add(1, nblk - 1, sd);
+            // the chains into the totals, in order
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) tot[m][r] += acc[m][r];
+                if (half == 1) {
+                    ex[m] = Y[m];                // the next k-part's e8m0 bytes
+                    refill(m, nblk - 1);
                 }
             }
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[r] = fmaf(Dc[r], sc_c, acc[r]);
-            if (i == kSubUnits - 1 || i == kBlkPerPart - 1) {
-                // end of a chain: into the total, in order
-#pragma unroll
-                for (int r = 0; r < 16; r++) tot[r] += acc[r];
-                acc = v16f{};
-            }
-            Dc = Dn;
-            sc_c = sc_n;
         }
-    };
-    for (int q = 0; q < P; q++) kpart(q, (q & 1) ? g_stage1 : g_stage0, (q & 1) ? g_stage0 : g_stage1);
-    // the caller's bias, loaded at its start, into LDS for its epilogue
-    if (threadIdx.x < nbias) bias_lds[threadIdx.x] = bias_v;
-    __syncthreads();             // callers reuse the LDS
-    return tot;
+    }
+    // the last direct loads (past the last k-part: zeros) land before the wave
+    // can end and its LDS be given away
+    __builtin_amdgcn_s_waitcnt(s_waitcnt_vm(0));
 }
 
 // ---- 5. grouped gate/up + SwiGLU-OAI + Q8 (+ image of h) ----
-// one workgroup per (token tile, group of 2 row tiles) (grouped_item); 4
-// waves: wave w = row tile w/2 of the group, gate (w even) or up (w odd).
+// one workgroup per (token tile, group of kGemmWaves row tiles)
+// (grouped_item); wave w: gate and up of row tile w of the group, so SwiGLU, the
+// Q8 and the image of a row tile finish in its wave.
 template <bool TRACE>
-__global__ __launch_bounds__(kGuThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_gateup_grouped(GroupedArgs a) {
+__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(TRACE ? 1 : 2))) void k_gateup_grouped(GroupedArgs a) {
+    constexpr int NW = kGemmWaves;
     __shared__ int src[32];
     const int T = a.dff / 32, P = a.parts_gu, nb = a.nb;
     int tile, grp;
-    if (!grouped_item(uniform(*a.ntiles), (T + 1) / 2, &tile, &grp)) return;
+    if (!grouped_item(uniform(*a.ntiles), (T + NW - 1) / NW, &tile, &grp)) return;
     const int4 tl = a.tiles[tile];
     const int e = uniform(tl.x), start = uniform(tl.y), cnt = uniform(tl.z);
     const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6));
-    const int rt = grp * 2 + (w >> 1), isup = w & 1;
+    const int rt = grp * NW + w;
     const bool live = rt < T;
-    if (threadIdx.x < 32) src[threadIdx.x] = (int)threadIdx.x < cnt ? a.sorted[start + threadIdx.x] / a.k : -1;
-    __syncthreads();
-    // the biases of the workgroup's 2 x (32 gate + 32 up) rows, requested now
-    // and kept in one register until the epilogue (a load issued after the
-    // GEMM would wait a full loaded-memory latency)
-    __shared__ float bias_s[128];                   // [row tile][gate 32 | up 32]
-    float bias_v = 0.0f;
-    {
-        const int t = (int)threadIdx.x, rtb = grp * 2 + (t >> 6), gu = (t >> 5) & 1;
-        const float* bp = gu ? a.up_b : a.gate_b;
-        if (t < 128 && bp && rtb < T) bias_v = bp[(size_t)e * a.dff + rtb * 32 + (t & 31)];
-    }
     const int ti = lane & 31, hb = lane >> 5;
     const bool valid = ti < cnt;
     const int pair = valid ? a.sorted[start + ti] : 0;
+    if (threadIdx.x < 32) src[threadIdx.x] = valid ? pair / a.k : -1;
+    // the biases of the row tile's 32 gate and 32 up rows, requested now and
+    // kept in one register until the epilogue (a load issued after the GEMM
+    // would wait a full loaded-memory latency)
+    __shared__ float bias_s[NW][64];
+    const float* bp = hb ? a.up_b : a.gate_b;
+    const float bias_v = bp && live ? bp[(size_t)e * a.dff + rt * 32 + ti] : 0.0f;
+    __syncthreads();
     WeightStream ws;
     {
         const size_t ex_units = (size_t)T * P * kUnits * 64;         // one expert's gate/up stream
         ws.rs = buf_rsrc(a.gu + (size_t)e * ex_units, (uint32_t)(ex_units * 16));
-        ws.off = (uint32_t)((((size_t)(live ? rt : T) * P) * kUnits * 64 + isup * 32 + (lane & 31)) * 16);
+        ws.off[0] = (uint32_t)((((size_t)(live ? rt : T) * P) * kUnits * 64 + ti) * 16);
+        ws.off[1] = ws.off[0] + 32 * 16;
         ws.ustride = 64 * 16;
-        ws.pstride = kUnits * 64 * 16;
     }
-    int32_t* tb = TRACE ? a.gu_sums + (((size_t)pair * 2 + isup) * a.dff + rt * 32) * nb : nullptr;
-
-    const v16f tot = grouped_parts<TRACE, kGuThreads>(ws, P, a.ximg, a.xsb, (size_t)a.n_tok, nb, src, lane, tb,
-                                          valid && live, bias_s, bias_v, 128);
-    // SwiGLU, Q8 and image of the row tile, split over its two waves: the
-    // lane's rows 8g + 4hb + c (g, c < 4) of groups g = isup and g = isup + 2
-    // are this wave's (so each wave owns whole hq words and whole 8-byte image
-    // runs); each wave hands the partner the totals of the partner's rows
-    // (LDS reused), then the block maximum is combined through LDS.
-    const int rtl = w >> 1;
-    float* xch = (float*)g_stage0;                // [row tile][sender][8][64]
-    float* mxs = xch + 2 * 2 * 8 * 64;            // [row tile][wave][64]
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int r = 4 * (1 - isup) + (j & 3) + 8 * (j >> 2);        // partner's j-th row
-        xch[((rtl * 2 + isup) * 8 + j) * 64 + lane] = tot[r];
+    int32_t* tb[2] = {nullptr, nullptr};
+    if (TRACE && valid && live) {
+        tb[0] = a.gu_sums + ((size_t)pair * 2 * a.dff + rt * 32) * nb;
+        tb[1] = tb[0] + (size_t)a.dff * nb;
     }
-    __syncthreads();
-    float hv[8], m = 0.0f;
+    v16f tot[2];
+    grouped_parts<TRACE, NW>(ws, P, a.ximg, a.xsb, (size_t)a.n_tok, nb, src, lane, tb, tot);
+    bias_s[w][lane] = bias_v;
+    wave_lds_order();                                                  // the wave's own row
+    if (!live) return;
+    // the lane's rows 8 g + 4 hb + c (g, c < 4): whole hq words, and with rows
+    // 16 apart (groups g and g + 2) whole 8-byte image runs
+    float hv[16], m = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int r = 4 * isup + (j & 3) + 8 * (j >> 2);                // this wave's j-th row
-        const int rr = 8 * (r >> 2) + 4 * hb + (r & 3);                 // row within the tile
-        const float own = tot[r], oth = xch[((rtl * 2 + 1 - isup) * 8 + j) * 64 + lane];
-        float vg = isup ? oth : own, vu = isup ? own : oth;
-        if (a.gate_b) vg += bias_s[rtl * 64 + rr];
-        if (a.up_b) vu += bias_s[rtl * 64 + 32 + rr];
+    for (int r = 0; r < 16; r++) {
+        const int rr = 8 * (r >> 2) + 4 * hb + (r & 3);
+        const float vg = tot[0][r] + bias_s[w][rr], vu = tot[1][r] + bias_s[w][32 + rr];   // zeros without biases
         const float xg = fminf(vg, a.limit);                           // engine_gpt2.rs:887-906
         const float yu = fminf(fmaxf(vu, -a.limit), a.limit);
-        hv[j] = (xg / (1.0f + expf(-a.alpha * xg))) * (yu + 1.0f);
-        m = fmaxf(m, fabsf(hv[j]));
+        hv[r] = (xg / (1.0f + expf(-a.alpha * xg))) * (yu + 1.0f);
+        m = fmaxf(m, fabsf(hv[r]));
     }
     m = fmaxf(m, __shfl_xor(m, 32));
-    mxs[(rtl * 2 + isup) * 64 + lane] = m;
-    __syncthreads();
-    m = fmaxf(m, mxs[(rtl * 2 + 1 - isup) * 64 + lane]);
     const float sc = fmaxf(1e-12f, m) / 127.0f;
-    if (!valid || !live) return;
-    // hq: the lane's groups g = isup, isup + 2 as 4-byte words; image: elements
-    // e and e + 16 sit at adjacent K (2e, 2e + 1), so groups g and g + 2 fill
-    // the 8 bytes K = 16 isup + 8hb .. +7 of each half
+    if (!valid) return;
     uint8_t* img = a.himg + ((size_t)pair * a.nbf + rt) * kImg;
-    // Q8 of the 8 values (the exact division only when some lane's quotient
-    // lies near a rounding tie), then the bytes: qw[gh] byte c = value
-    // j = 4 gh + c; the image run's byte 2 (c & 1) + gh of word c >> 1 holds
-    // value j's 16h (hi) and l (lo) as e4m3, whose hardware conversion is
-    // exact for these integers (|16h| <= 128, 0 <= l <= 15)
-    int qv[8];
+    // Q8 of the values (the exact division only when some lane's quotient lies
+    // near a rounding tie), then the bytes: qw[g] byte c = value 4 g + c; elements
+    // e and e + 16 sit at adjacent K (2e, 2e + 1), so groups g and g + 2 fill the
+    // 8 bytes K = 16 g + 8 hb .. +7 (g < 2) of each half: byte 2 (c & 1) + (0 for
+    // g, 1 for g + 2) of word c >> 1 holds the value's 16h (hi) and l (lo) as
+    // e4m3, whose hardware conversion is exact for these integers (|16h| <= 128, 0
+    // <= l <= 15)
+    int qv[16];
     {
         const float rs = __builtin_amdgcn_rcpf(sc);
-        float r[8];
+        float r[16];
         bool near = false;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < 16; j++) {
             const float y = hv[j] * rs;
             r[j] = __builtin_rintf(y);
             near = near || q8_near_half(y);
         }
         if (near) {
 #pragma unroll
-            for (int j = 0; j < 8; j++)
+            for (int j = 0; j < 16; j++)
                 if (q8_near_half(hv[j] * rs)) r[j] = roundf(hv[j] / sc);
         }
 #pragma unroll
-        for (int j = 0; j < 8; j++) qv[j] = q8_clamp(r[j]);
+        for (int j = 0; j < 16; j++) qv[j] = q8_clamp(r[j]);
     }
-    uint32_t qw[2] = {0u, 0u}, hi[2], lo[2];
+    uint32_t* hqw = (uint32_t*)(a.hq + (size_t)pair * a.dff + rt * 32 + 4 * hb);
 #pragma unroll
-    for (int j = 0; j < 8; j++) qw[j >> 2] |= ((uint32_t)qv[j] & 0xffu) << (8 * (j & 3));
-    float fh[8], fl[8];
+    for (int g = 0; g < 4; g++) {
+        uint32_t qw = 0u;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+        for (int c = 0; c < 4; c++) qw |= ((uint32_t)qv[4 * g + c] & 0xffu) << (8 * c);
+        hqw[2 * g] = qw;
+    }
+    float fh[16], fl[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
         const int h = qv[j] >> 4;
         fh[j] = (float)(16 * h);
         fl[j] = (float)(qv[j] - 16 * h);
     }
 #pragma unroll
-    for (int w2 = 0; w2 < 2; w2++) {
-        // word w2: bytes (c = 2 w2, gh 0), (c = 2 w2, gh 1), (c = 2 w2 + 1, gh 0), (c = 2 w2 + 1, gh 1)
-        const int c0 = 2 * w2, c1 = 2 * w2 + 1;
-        hi[w2] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(fh[c1], fh[4 + c1],
-                                                            __builtin_amdgcn_cvt_pk_fp8_f32(fh[c0], fh[4 + c0], 0, false), true);
-        lo[w2] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(fl[c1], fl[4 + c1],
-                                                            __builtin_amdgcn_cvt_pk_fp8_f32(fl[c0], fl[4 + c0], 0, false), true);
+    for (int g = 0; g < 2; g++) {
+        uint32_t hi[2], lo[2];
+#pragma unroll
+        for (int w2 = 0; w2 < 2; w2++) {
+            // word w2: values (g, c0), (g + 2, c0), (g, c0 + 1), (g + 2, c0 + 1), c0 = 2 w2
+            const int j0 = 4 * g + 2 * w2, j1 = j0 + 8;
+            hi[w2] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(fh[j0 + 1], fh[j1 + 1], __builtin_amdgcn_cvt_pk_fp8_f32(fh[j0], fh[j1], 0, false), true);
+            lo[w2] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(fl[j0 + 1], fl[j1 + 1], __builtin_amdgcn_cvt_pk_fp8_f32(fl[j0], fl[j1], 0, false), true);
+        }
+        *(uint2*)(img + 32 * g + 8 * hb) = make_uint2(hi[0], hi[1]);
+        *(uint2*)(img + 32 * g + 8 * hb + 16) = make_uint2(lo[0], lo[1]);
     }
-    uint32_t* hqw = (uint32_t*)(a.hq + (size_t)pair * a.dff + rt * 32 + 8 * isup + 4 * hb);
-    hqw[0] = qw[0];
-    hqw[4] = qw[1];
-    *(uint2*)(img + 32 * isup + 8 * hb) = make_uint2(hi[0], hi[1]);
-    *(uint2*)(img + 32 * isup + 8 * hb + 16) = make_uint2(lo[0], lo[1]);
-    if (hb == 0 && !isup) a.hsb[(size_t)pair * a.nbf + rt] = sc;
+    if (hb == 0) a.hsb[(size_t)pair * a.nbf + rt] = sc;
 }
 
 // ---- 6. grouped down (+ bias) into dnout ----
-// one workgroup per (token tile, group of 8 row tiles of 32 rows) (grouped_item).
+// one workgroup per (token tile, group of 2 kGemmWaves row tiles of 32 rows)
+// (grouped_item); wave w: row tiles 2 w and 2 w + 1 of the group.
 template <bool TRACE>
-__global__ __launch_bounds__(kDnThreads) void k_down_grouped(GroupedArgs a) {
+__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(TRACE ? 1 : 2))) void k_down_grouped(GroupedArgs a) {
+    constexpr int NW = kGemmWaves;
     __shared__ int src[32];
     int tile, grp;
-    if (!grouped_item(uniform(*a.ntiles), (a.d / 32 + 7) / 8, &tile, &grp)) return;
+    const int T = a.d / 32;
+    if (!grouped_item(uniform(*a.ntiles), (T + 2 * NW - 1) / (2 * NW), &tile, &grp)) return;
     const int4 tl = a.tiles[tile];
     const int e = uniform(tl.x), start = uniform(tl.y), cnt = uniform(tl.z);
     const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6));
     const int RTv = mx_down_rt(a.k), Tv = a.d / RTv, P = a.parts_dn, nbf = a.nbf;
-    const int rt = grp * 8 + w;
-    const bool live = rt < a.d / 32;
-    if (threadIdx.x < 32) src[threadIdx.x] = (int)threadIdx.x < cnt ? a.sorted[start + threadIdx.x] : -1;
-    __syncthreads();
+    const int rt = grp * 2 * NW + 2 * w;
     const int ti = lane & 31, hb = lane >> 5;
     const bool valid = ti < cnt;
     const int pair = valid ? a.sorted[start + ti] : 0;
-    const int row_l = rt * 32 + (lane & 31);                          // this lane's A row
-    // the biases of the workgroup's 8 x 32 rows, requested now (one register
-    // until the epilogue)
-    __shared__ float bias_s[256];
-    float bias_v = 0.0f;
-    if (threadIdx.x < 256 && a.down_b && grp * 256 + (int)threadIdx.x < a.d)
-        bias_v = a.down_b[(size_t)e * a.d + grp * 256 + threadIdx.x];
+    if (threadIdx.x < 32) src[threadIdx.x] = valid ? pair : -1;
+    // the biases of the wave's 64 rows, requested now (one register until the
+    // epilogue)
+    __shared__ float bias_s[NW][64];
+    const float bias_v = a.down_b && rt * 32 + lane < a.d ? a.down_b[(size_t)e * a.d + rt * 32 + lane] : 0.0f;
+    __syncthreads();
     WeightStream ws;
     {
         const size_t ex_units = (size_t)Tv * P * kUnits * RTv;      // one expert's down stream
         ws.rs = buf_rsrc(a.dn + (size_t)e * ex_units, (uint32_t)(ex_units * 16));
-        ws.off = live ? (uint32_t)(((size_t)(row_l / RTv) * P * kUnits * RTv + row_l % RTv) * 16) : kOffNone;
-        ws.ustride = RTv * 16;
-        ws.pstride = kUnits * RTv * 16;
-    }
-    int32_t* tb = TRACE ? a.dn_sums + ((size_t)pair * a.d + rt * 32) * nbf : nullptr;
-
-    const v16f tot = grouped_parts<TRACE, kDnThreads>(ws, P, a.himg, a.hsb, (size_t)a.n_tok * a.k, nbf, src, lane,
-                                          tb, valid && live, bias_s, bias_v, 256);
-    if (!valid || !live) return;
-    float* out = a.dnout + (size_t)pair * a.d + rt * 32 + 4 * hb;
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        float4 v;
-        float* vp = (float*)&v;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int row = rt * 32 + 8 * g + 4 * hb + c;
-            vp[c] = tot[4 * g + c] + (a.down_b ? bias_s[row - grp * 256] : 0.0f);
+        for (int m = 0; m < 2; m++) {
+            const int row_l = (rt + m) * 32 + ti;                    // the lane's A row
+            ws.off[m] = rt + m < T ? (uint32_t)(((size_t)(row_l / RTv) * P * kUnits * RTv + row_l % RTv) * 16) : kOffNone;
         }
-        *(float4*)(out + 8 * g) = v;
+        ws.ustride = RTv * 16;
+    }
+    int32_t* tb[2] = {nullptr, nullptr};
+    if (TRACE && valid) {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+            if (rt + m < T) tb[m] = a.dn_sums + ((size_t)pair * a.d + (rt + m) * 32) * nbf;
+    }
+    v16f tot[2];
+    grouped_parts<TRACE, NW>(ws, P, a.himg, a.hsb, (size_t)a.n_tok * a.k, nbf, src, lane, tb, tot);
+    bias_s[w][lane] = bias_v;
+    wave_lds_order();                                                // the wave's own row
+    if (!valid) return;
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        if (rt + m >= T) break;
+        float* out = a.dnout + (size_t)pair * a.d + (rt + m) * 32 + 4 * hb;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            float4 v;
+            float* vp = (float*)&v;
+#pragma unroll
+            for (int c = 0; c < 4; c++) vp[c] = tot[m][4 * g + c] + bias_s[w][m * 32 + 8 * g + 4 * hb + c];   // zeros without biases
+            *(float4*)(out + 8 * g) = v;
+        }
     }
 }
 
@@ -950,14 +1003,15 @@ int launch_grouped_layer(const GroupedArgs& a, bool trace, hipStream_t s, const 
     }
     // one workgroup per (token tile, row group), dealt out by grouped_item:
     // 8 slots per XCD round, enough for the largest tile count
-    const int ngu = a.max_tiles * ((a.dff / 32 + 1) / 2), ndn = a.max_tiles * ((a.d / 32 + 7) / 8);
+    const int ngu = a.max_tiles * ((a.dff / 32 + kGemmWaves - 1) / kGemmWaves);
+    const int ndn = a.max_tiles * ((a.d / 32 + 2 * kGemmWaves - 1) / (2 * kGemmWaves));
     const dim3 ggu((ngu + 7) / 8 * 8), gdn((ndn + 7) / 8 * 8);
     if (ev) armed_events() = ev[0];
-    if (trace) launch(k_gateup_grouped<true>, ggu, dim3(kGuThreads), 0, s, a);
-    else launch(k_gateup_grouped<false>, ggu, dim3(kGuThreads), 0, s, a);
+    if (trace) launch(k_gateup_grouped<true>, ggu, dim3(64 * kGemmWaves), 0, s, a);
+    else launch(k_gateup_grouped<false>, ggu, dim3(64 * kGemmWaves), 0, s, a);
     if (ev) armed_events() = ev[1];
-    if (trace) launch(k_down_grouped<true>, gdn, dim3(kDnThreads), 0, s, a);
-    else launch(k_down_grouped<false>, gdn, dim3(kDnThreads), 0, s, a);
+    if (trace) launch(k_down_grouped<true>, gdn, dim3(64 * kGemmWaves), 0, s, a);
+    else launch(k_down_grouped<false>, gdn, dim3(64 * kGemmWaves), 0, s, a);
     launch(k_combine_batch, dim3((unsigned)std::min<size_t>(((size_t)nt * (a.d / 4) + 255) / 256, 2048)), dim3(256), 0, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -19;
 }

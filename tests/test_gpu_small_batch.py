@@ -67,3 +67,18 @@ def test_batched_selection_ties(gpu, ne, k, n_tok):
     W[1] = W[2] = W[0]                               # and one four times
     X = np.stack([synth.token(384, 23, i) for i in range(n_tok)])
     check(L, MoeConfig.gptoss(d=384, n_expert=ne, top_k=k, d_ff=64, max_tokens=n_tok), X, "gptoss")
+
+
+# the matrix-core tiles: k-parts of 15 blocks cut short in either sub-part, row tiles that are no
+# whole workgroup in gate/up (4) and down (8), several tiles per expert
+@pytest.mark.parametrize("d,dff,ne,k,n_tok", [
+    (32 * 15, 32 * 16, 4, 2, 70),
+    (32 * 16, 32 * 23, 4, 4, 33),
+    (32 * 31, 32 * 5, 8, 4, 65),
+    (32 * 24, 32 * 30, 3, 3, 40),
+])
+def test_mxfp4_tiles(gpu, d, dff, ne, k, n_tok):
+    print(f"case tiles d={d} dff={dff} ne={ne} k={k} n_tok={n_tok}", flush=True)
+    L = synth.gptoss_layer(d, dff, ne, k, seed=24, zipf=1.1)
+    X = np.stack([synth.token(d, 24, i) for i in range(n_tok)])
+    check(L, MoeConfig.gptoss(d=d, n_expert=ne, top_k=k, d_ff=dff, max_tokens=n_tok), X, "gptoss")
