@@ -37,6 +37,7 @@
 #include "cpb_internal.h"
 #include "moe_common.h"
 #include "route_dev.h"
+#include "select.h"
 
 namespace cpb {
 
@@ -455,8 +456,6 @@ __global__ __launch_bounds__(1024) void k_head_refine(HeadDev a) {
     __shared__ __align__(16) int rsi[kRefineWaves][64];
     __shared__ __align__(16) uint64_t rsk[kRefineWaves][64];
     __shared__ int cid[kHeadMaxCand];
-    __shared__ float lgs[128];
-    __shared__ int ids_s[128];
     __shared__ int last;
     const int w = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int i = tid; i < nb * 8; i += 1024) xl[i] = ((const uint32_t*)a.xq)[i];
@@ -466,9 +465,18 @@ __global__ __launch_bounds__(1024) void k_head_refine(HeadDev a) {
     const int M = r0 == r1 ? 0 : ((r1 - 1) / kHeadGroupRows - a.wtab[2 * w] + 1) * C;
     const float* cv = a.candv + a.wtab[2 * w + 1];
     const int* ci = a.candi + a.wtab[2 * w + 1];
-    // each wave: chunks of 64 entries by rank, folded into a running best n_cand
-    {
-        const int nchunk = (M + 63) / 64;
+    const int nchunk = (M + 63) / 64;
+    if (nchunk <= kRefineWaves) {
+        // one chunk of 64 entries per wave: its best n_cand by rank
+        const int e = wave * 64 + lane;
+        const float v = e < M ? cv[e] : -INFINITY;
+        const int i = e < M ? ci[e] : INT32_MAX;
+        const int rank = wave_rank(v, i, rsk[wave]);
+        if (i != INT32_MAX && rank < C) { wv[wave][rank] = v; wi[wave][rank] = i; }
+        const int n_real = __builtin_popcountll(__ballot(i != INT32_MAX));
+        if (lane >= n_real && lane < C) { wv[wave][lane] = -INFINITY; wi[wave][lane] = INT32_MAX; }
+    } else {
+        // each wave: chunks by rank, folded into a running best n_cand
         float runv = -INFINITY;
         int runi = INT32_MAX;                 // lane k < C: the wave's k-th best so far
         for (int ch = wave; ch < nchunk; ch += kRefineWaves) {
@@ -580,21 +588,28 @@ __global__ __launch_bounds__(1024) void k_head_refine(HeadDev a) {
     }
     __syncthreads();
     if (!last) return;
+    // the first of the largest (the reference's scan with a strict comparison,
+    // from -FLT_MAX and row 0: a NaN or -FLT_MAX never wins): wave 0, two of the
+    // at most 128 candidates per lane, the largest by order-preserving keys and
+    // the lowest index by ballot.  This in place of a scan by one thread, and one
+    // ranking instead of two above: 14.6 -> 9.3 us (201088 rows, 12 workers)
+    if (wave) return;
     const int nc = a.nt * C;
-    if (tid < nc) {
-        lgs[tid] = ld_dev(a.cand_logits + tid);
-        ids_s[tid] = ld_dev(a.cand_ids + tid);
+    uint32_t key[2];
+    int id[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int k = lane + 64 * j;
+        const float v = k < nc ? ld_dev(a.cand_logits + k) : -INFINITY;
+        id[j] = k < nc ? ld_dev(a.cand_ids + k) : 0;
+        key[j] = v > -FLT_MAX ? float_key(v + 0.0f) : 0u;            // -0 and +0 are equal
     }
-    __syncthreads();
-    if (tid == 0) {
-        float best = -FLT_MAX;
-        int bi = 0;
-        for (int k = 0; k < nc; k++)
-            if (lgs[k] > best) { best = lgs[k]; bi = ids_s[k]; }
-        *a.chosen = bi;
-    }
+    const uint32_t m = wave_max_u32(max(key[0], key[1]));
+    const uint64_t b0 = __ballot(key[0] == m), b1 = __ballot(key[1] == m);
+    const int src = __builtin_ctzll(b0 ? b0 : b1);
+    const int bi = __builtin_amdgcn_readlane(b0 ? id[0] : id[1], src);
+    if (lane == 0) *a.chosen = m ? bi : 0;
 }
-
 // LDS of k_head_refine: candidate rows and scales, activations
 inline size_t head_refine_lds(int d, int nc) { return (size_t)nc * d + (size_t)nc * (d / 32) * 4 + (size_t)(d / 32) * 36; }
 
