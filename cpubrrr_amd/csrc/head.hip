@@ -440,6 +440,9 @@ __global__ __launch_bounds__(256) void k_head_screen(HeadDev a) {
 // row order), their exact Q8 logits (dot_q8_i8, :169-191), then the greedy
 // choice over all workers' candidates in worker / rank order (:128-134) by the
 // last workgroup to finish.  grid: n_slices workgroups of 1024 threads.
+// A chain of short dependent phases (12 workgroups; 201088 rows, 14.6 -> 9.3 us
+// with the lists ranked in one pass where a slice has at most 16 chunks of them,
+// and the choice over the candidates by the first wave's keys in registers).
 constexpr int kRefineWaves = 16;
 __global__ __launch_bounds__(1024) void k_head_refine(HeadDev a) {
     extern __shared__ __align__(16) unsigned char smem[];

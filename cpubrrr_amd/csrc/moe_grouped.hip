@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64) void k_router_exact(GroupedArgs a) {
 // The same for batches that leave most of the chip idle, where a chain's
 // length is the kernel's time: workgroup = 16 experts x 4 tokens, whose 64
 // chains are wave 0's lanes (lane 16 r + i: expert 16 ex + i, token 4 ty + r).
-// Wave 0 only adds; four producer waves form the products a chunk of 128 steps
+// Wave 0 only adds; two producer waves form the products a chunk of 128 steps
 // ahead, in LDS as wave 0 reads them ([4 steps][lane], 16 bytes).  A
 // producer's unit is 16 steps: its lane 16 r + i holds expert i's row at steps
 // 4 r .. 4 r + 3 (one 1 KB load of the transposed copy, nothing twice) and
@@ -374,6 +374,9 @@ int launch_router_transpose(const float* w, float* out, int ne, int d, hipStream
 // them: lane l holds experts l + 64 j as order-preserving 32-bit keys, K
 // rounds of a wave maximum, the lowest index by ballot.  A NaN ranks last (a
 // strict comparison never lets one in), as -inf.
+// Bound by the rounds' chain in the wave, so four tokens share a workgroup to
+// put all of them in flight at once: 512 tokens x 32 experts 4.8 us, where
+// decode's selector with its intervals and certificate took 22.
 struct TokenLogits {
     float v[4];
 };
@@ -487,7 +490,11 @@ __global__ __launch_bounds__(1024) void k_group_scan(GroupedArgs a) {
     group_pairs<kScanPer>(a, ex);
 }
 // Small batches: selection and grouping in one launch, a wave per kSelTok
-// tokens (16 waves; np <= 1024)
+// tokens (16 waves; np <= 1024).  One workgroup's four rounds of selection cost
+// less than a launch and its gap at few tokens (3 tokens 9.3 -> 4.0 us) and the
+// same at 64 (whole layer of 32 experts, 128.3 us at 64 tokens fused, 127.4 at 65
+// in two launches); beyond, its waves would rank more tokens in turn while the
+// chip stands idle.
 constexpr int kSelTok = 4, kSelMax = 16 * kSelTok;
 __global__ __launch_bounds__(1024) void k_select_group(GroupedArgs a) {
     __shared__ int ids_l[kSelMax * 8];
@@ -639,7 +646,9 @@ CPB_DEV void mfma_gap() { asm volatile("s_nop 7"); }
 // wave, whose activations both tiles' products read from LDS once (a b128 read
 // takes the LDS 16 cycles, so at one tile per read the four SIMDs' reads took
 // 61 ns per block and tile against 28 of matrix-core and 27 of VALU work: two,
-// three and four waves per SIMD all ran at that rate).  Per
+// three and four waves per SIMD all ran at that rate).  512 tokens x 32
+// experts: gate/up 161 -> 149 us, down 87 -> 76; 2049 x 128: 574 -> 496 and
+// 298 -> 255.  Now reads, fmas and products take about the same time.  Per
 // block, D = A(rows) x B(tokens) on the matrix cores and acc = fma(D, xsb, acc)
 // in block order, in two chains per k-part (its sub-parts, as the decode
 // kernels' two wavefronts per k-part), the chains added to the total in order.
