@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64) void k_router_exact(GroupedArgs a) {
 // The same for batches that leave most of the chip idle, where a chain's
 // length is the kernel's time: workgroup = 16 experts x 4 tokens, whose 64
 // chains are wave 0's lanes (lane 16 r + i: expert 16 ex + i, token 4 ty + r).
-// Wave 0 only adds; two producer waves form the products a chunk of 128 steps
+// Wave 0 only adds; two producer waves form the products a chunk of CHUNK steps
 // ahead, in LDS as wave 0 reads them ([4 steps][lane], 16 bytes).  A
 // producer's unit is 16 steps: its lane 16 r + i holds expert i's row at steps
 // 4 r .. 4 r + 3 (one 1 KB load of the transposed copy, nothing twice) and
@@ -231,21 +231,23 @@ __global__ __launch_bounds__(64) void k_router_exact(GroupedArgs a) {
 // 26.5 -> 17.1, 11 tokens x 128 experts x 2048 17.3 -> 11.5 us against
 // k_router_exact.  Every lane reading its own 16 bytes of both operands
 // instead (no exchange) was bound by the L1: four lanes in four read the same.
-constexpr int kPcChunk = 128, kPcProducers = 2, kPcAhead = 6;      // chunks requested ahead
-constexpr int kPcQ = kPcChunk / 4;                // 16-byte units of a chain's chunk
+constexpr int kPcProducers = 2, kPcSteps = 768;   // steps requested ahead
 template <int S>
 CPB_DEV float row_bcast(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + S, 0xf, 0xf, true));
 }
+template <int CHUNK>
 __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(GroupedArgs a) {
-    constexpr int UP = kPcChunk / 16 / kPcProducers;   // a producer's units per chunk
+    constexpr int kPcAhead = kPcSteps / CHUNK, kPcQ = CHUNK / 4;      // chunks requested ahead; 16-byte units of a chain's chunk
+    constexpr int UP = CHUNK / 16 / kPcProducers;     // a producer's units per chunk
+    constexpr int B = CHUNK / 32;                     // its blocks of 8 units
     static_assert(kPcAhead % 3 == 0, "the register sets and the LDS buffers turn together");
     __shared__ __align__(16) f32x4 prod[3][kPcQ][64];
     const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6)), d = a.d, nt = a.n_tok, ne = a.ne;
     const int i = lane & 15, r = lane >> 4, e = blockIdx.x * 16 + i, t = blockIdx.y * 4 + r;
     // whole rounds of the register sets (the barriers of every wave; chunks past
     // the row's end are formed from other values or zeros and not summed)
-    const int nch = (d + kPcAhead * kPcChunk - 1) / (kPcAhead * kPcChunk) * kPcAhead;
+    const int nch = (d + kPcAhead * CHUNK - 1) / (kPcAhead * CHUNK) * kPcAhead;
     if (w) {
         const __amdgpu_buffer_rsrc_t rx = buf_rsrc(a.xn, (uint32_t)((size_t)nt * d * 4));
         const __amdgpu_buffer_rsrc_t rw = buf_rsrc(a.router_t, (uint32_t)((size_t)router_t_rows(ne) * d * 4));
@@ -258,7 +260,7 @@ __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(
         // (the whole offset in the vector offset: the scalar one is not part
         // of the buffer's range check)
         auto load = [&](int s, int ch) {
-            const uint32_t wc = wo + (uint32_t)ch * (kPcChunk * 64), xc = xo + (uint32_t)ch * (kPcChunk * 4);
+            const uint32_t wc = wo + (uint32_t)ch * (CHUNK * 64), xc = xo + (uint32_t)ch * (CHUNK * 4);
 #pragma unroll
             for (int u = 0; u < UP; u++) {
                 wv[s][u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wc + u * 1024, 0, 0));
@@ -311,7 +313,7 @@ __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(
         asm volatile("" ::: "memory");
     };
     float acc = (a.router_b && e < ne) ? a.router_b[e] : 0.0f;
-    const int nb = d / 32;                        // blocks of 8 units (d % 32 == 0), 4 per chunk
+    const int nb = d / 32;                        // blocks of 8 units (d % 32 == 0), B per chunk
     f32x4 v[8];
     auto block = [&](const f32x4* nx) {           // sums the 8 units in v, reads the next 8
 #pragma unroll
@@ -329,24 +331,24 @@ __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(
         }
     };
     // block m's successor in buffer j: this chunk's, or the first of the next chunk, which is complete
-    auto next = [&](int j, int m) { return m < 3 ? &prod[j][8 * (m + 1)][lane] : &prod[(j + 1) % 3][0][lane]; };
+    auto next = [&](int j, int m) { return m < B - 1 ? &prod[j][8 * (m + 1)][lane] : &prod[(j + 1) % 3][0][lane]; };
     int k = 0;
     arrive();
 #pragma unroll
     for (int u = 0; u < 8; u++) v[u] = prod[0][u][lane];
-    for (; 4 * (k + 3) <= nb; k += 3) {
+    for (; B * (k + 3) <= nb; k += 3) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
 #pragma unroll
-            for (int m = 0; m < 4; m++) block(next(j, m));
+            for (int m = 0; m < B; m++) block(next(j, m));
             arrive();                             // of the next chunk
         }
     }
 #pragma unroll
     for (int j = 0; j < 3; j++) {
 #pragma unroll
-        for (int m = 0; m < 4; m++)
-            if (4 * (k + j) + m < nb) block(next(j, m));
+        for (int m = 0; m < B; m++)
+            if (B * (k + j) + m < nb) block(next(j, m));
         if (k + j + 1 < nch) arrive();
     }
     for (k += 4; k < nch; k++) arrive();          // the producers' last rounds
@@ -995,9 +997,14 @@ int launch_grouped_layer(const GroupedArgs& a, bool trace, hipStream_t s, const 
         launch(k_prep_batch, dim3(nt), dim3(256), sizeof(float) * (2 * a.d + 64), s, a);
     }
     const int et = router_t_rows(a.ne) / 16, rt = (nt + 3) / 4;
-    // one workgroup of 96 KB LDS per CU: a second round would cost what
-    // k_router_exact takes (777 tokens x 128 experts: 27 us there)
-    if (et * rt <= 256) launch(k_router_exact_small, dim3(et, rt), dim3(64 * (1 + kPcProducers)), 0, s, a);
+    // One workgroup of 96 KB LDS per CU; up to two per CU with chunks of half
+    // the length (48 KB, twice the barriers; whole layer, 128 experts top-8: 132
+    // tokens 174.9 -> 170.7 us, 256 tokens 184.2 -> 179.5; 32 experts: 600 tokens
+    // 273.3 -> 266.7, 1000 tokens 373.1 -> 367 us against k_router_exact).  Three
+    // per CU share the SIMDs' issue: 384 x 128 207.2 -> 206.0, 1536 x 32 514.8 ->
+    // 518, so k_router_exact takes those and the larger.
+    if (et * rt <= 256) launch(k_router_exact_small<128>, dim3(et, rt), dim3(64 * (1 + kPcProducers)), 0, s, a);
+    else if (et * rt <= 512) launch(k_router_exact_small<64>, dim3(et, rt), dim3(64 * (1 + kPcProducers)), 0, s, a);
     else launch(k_router_exact, dim3((a.ne + 7) / 8, (nt + 7) / 8), dim3(64), 0, s, a);
     if (nt <= kSelMax) {
         launch(k_select_group, dim3(1), dim3(1024), 0, s, a);

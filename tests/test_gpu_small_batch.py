@@ -29,8 +29,12 @@ def check(L, cfg, X, family):
     (416, 64, 20, 4, 3),        # 13 blocks, 20 experts
     (3840, 64, 33, 3, 5),       # the longest row, 33 experts
     (1088, 96, 16, 1, 17),
-    (448, 64, 128, 4, 128),     # the last size of the small batch's router kernel
-    (448, 64, 128, 4, 129),     # the first of the other
+    (448, 64, 128, 4, 128),     # the last size of the small batch's router kernel in long chunks
+    (448, 64, 128, 4, 129),     # the first in short chunks
+    (416, 64, 120, 2, 137),     # 13 blocks, half a chunk at the end, experts and tokens that are no whole groups
+    (1568, 64, 128, 2, 133),    # more than the steps requested ahead
+    (448, 64, 128, 4, 256),     # the last in short chunks
+    (448, 64, 128, 4, 257),     # the first of the other kernel
 ])
 def test_mxfp4_small_batches(gpu, d, dff, ne, k, n_tok):
     print(f"case small batch d={d} dff={dff} ne={ne} k={k} n_tok={n_tok}", flush=True)
