@@ -52,6 +52,26 @@ CPB_DEV uint32_t img_hi(uint32_t v) {
 CPB_DEV uint32_t img_lo(uint32_t v) {
     return nib_lookup<0>(v, table4(img_l_entry, 0), table4(img_l_entry, 1), table4(img_l_entry, 2), table4(img_l_entry, 3));
 }
+// To be called on a matrix product's result before anything else uses it.  The
+// hardware does not hold an instruction back that reads an MFMA's result too
+// early: passes + 4 issue states have to lie between (20 for the 32 x 32 x 64
+// f8f6f4 product, 12 for the others here).  The compiler pads to that, but it
+// counts an s_waitcnt as a state, and one that is already satisfied takes none:
+// without this, uses came up to two states early (sums of the grouped MXFP4
+// GEMMs' last blocks were wrong on every run).  The result passes through the
+// asm, so no use can move before it, and the compiler does not count the asm:
+// its two states come on top.  tests/test_mfma_results.py counts them in the
+// assembly.
+template <typename V>
+CPB_DEV void mfma_result(V& D) {
+    asm("s_nop 1" : "+v"(D));
+}
+// The whole wait in place: nothing the compiler adds (a spill or a copy of the
+// result before its use) can come too early either.
+template <typename V>
+CPB_DEV void mfma_result_now(V& D) {
+    asm("s_nop 15\n\ts_nop 3" : "+v"(D));
+}
 CPB_DEV int sdot4(uint32_t a, uint32_t b, int c) { return __builtin_amdgcn_sdot4((int)a, (int)b, c, false); }
 
 // 2^(e-128) * xsb exactly as the reference computes tbl[e] * xsb, with tbl

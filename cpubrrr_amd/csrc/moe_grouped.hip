@@ -638,12 +638,6 @@ CPB_DEV void split_pair(const u32x4& v, u32x4& x, u32x4& y) {
     }
 }
 
-// A 16-pass MFMA's results may be read 19 wait states after it.  Where only the
-// other tile's sixteen fmas, one MFMA and waits lie between, the compiler left
-// 17 (the last blocks' sums were read too early, wrong on every run): mfma_gap
-// adds 8 there.  Elsewhere at least three LDS reads lie between as well.
-CPB_DEV void mfma_gap() { asm volatile("s_nop 7"); }
-
 // The loop shared by the two grouped GEMMs: two row tiles x one token tile per
 // wave, whose activations both tiles' products read from LDS once (a b128 read
 // takes the LDS 16 cycles, so at one tile per read the four SIMDs' reads took
@@ -728,6 +722,7 @@ CPB_DEV void grouped_parts(const WeightStream& ws, int P, const uint8_t* img, co
             };
             auto add = [&](int m, int i, float s) {
                 if (TRACE) trace(m, i);
+                else mfma_result(D[m]);
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[m][r] = fmaf(D[m][r], s, acc[m][r]);
             };
@@ -738,6 +733,7 @@ CPB_DEV void grouped_parts(const WeightStream& ws, int P, const uint8_t* img, co
                 const int bl = half * kSub + i;
                 if (!(i & 1)) split_pair(wp[m][half * 4 + (i >> 1)], X[m], Y[m]);
                 D[m] = mx_block_mfma_b(i & 1 ? Y[m] : X[m], xa[i & 1][0], xa[i & 1][1], ex[m][bl >> 2], bl);
+                if (TRACE) mfma_result_now(D[m]);        // these kernels spill, results among what they spill
                 if (i & 1) refill(m, i);
             };
             xread(0);
@@ -747,20 +743,15 @@ CPB_DEV void grouped_parts(const WeightStream& ws, int P, const uint8_t* img, co
                 mul(0, i);
                 // keep the order as written
                 __builtin_amdgcn_sched_barrier(0);
-                if (i) {
-                    if (i + 1 >= nblk) mfma_gap();
-                    add(1, i - 1, sd);
-                }
+                if (i) add(1, i - 1, sd);
                 __builtin_amdgcn_sched_barrier(0);
                 mul(1, i);
                 sd = sa[i & 1];
                 if (i + 2 < nblk) xread(i + 2);
                 __builtin_amdgcn_sched_barrier(0);
-                if (i + 2 >= nblk) mfma_gap();
                 add(0, i, sd);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            mfma_gap();
             add(1, nblk - 1, sd);
             // the chains into the totals, in order
 #pragma unroll
@@ -784,7 +775,7 @@ CPB_DEV void grouped_parts(const WeightStream& ws, int P, const uint8_t* img, co
 // (grouped_item); wave w: gate and up of row tile w of the group, so SwiGLU, the
 // Q8 and the image of a row tile finish in its wave.
 template <bool TRACE>
-__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(TRACE ? 1 : 2))) void k_gateup_grouped(GroupedArgs a) {
+__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(2))) void k_gateup_grouped(GroupedArgs a) {
     constexpr int NW = kGemmWaves;
     __shared__ int src[32];
     const int T = a.dff / 32, P = a.parts_gu, nb = a.nb;
@@ -901,7 +892,7 @@ __global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu
 // one workgroup per (token tile, group of 2 kGemmWaves row tiles of 32 rows)
 // (grouped_item); wave w: row tiles 2 w and 2 w + 1 of the group.
 template <bool TRACE>
-__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(TRACE ? 1 : 2))) void k_down_grouped(GroupedArgs a) {
+__global__ __launch_bounds__(64 * kGemmWaves) __attribute__((amdgpu_waves_per_eu(2))) void k_down_grouped(GroupedArgs a) {
     constexpr int NW = kGemmWaves;
     __shared__ int src[32];
     int tile, grp;

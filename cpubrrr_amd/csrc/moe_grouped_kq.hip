@@ -258,16 +258,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         int sumi[16];
+        uint2 sm[16];                            // the rows' eight scales
 #pragma unroll
-        for (int i = 0; i < 16; i++) sumi[i] = 0;
+        for (int i = 0; i < 16; i++) {
+            sumi[i] = 0;
+            sm[i] = *(const uint2*)&s_sm[w][d_row(i, hb)][0];
+        }
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
-            const v16i_k D0 = mfma_i8(and4(wq[jj], 0x0F0F0F0Fu), xb[2 * jj]);
-            const v16i_k D1 = mfma_i8(and4(shr4(wq[jj], 4), 0x0F0F0F0Fu), xb[2 * jj + 1]);
+            v16i_k D0 = mfma_i8(and4(wq[jj], 0x0F0F0F0Fu), xb[2 * jj]);
+            v16i_k D1 = mfma_i8(and4(shr4(wq[jj], 4), 0x0F0F0F0Fu), xb[2 * jj + 1]);
+            mfma_result(D0);
+            mfma_result(D1);
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int row = d_row(i, hb);
-                sumi[i] += mul24(D0[i], (int)s_sm[w][row][2 * jj]) + mul24(D1[i], (int)s_sm[w][row][2 * jj + 1]);
+                const uint32_t s2 = (jj < 2 ? sm[i].x : sm[i].y) >> (16 * (jj & 1));
+                sumi[i] += mul24(D0[i], (int)(s2 & 0xffu)) + mul24(D1[i], (int)((s2 >> 8) & 0xffu));
             }
         }
         // mint = sum_j mn[row][j] * xs8[tok][j] on the matrix cores: xs8 =
@@ -287,6 +293,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             const uint2 zero = {0u, 0u}, B = {bw[0], bw[1]};
             M1 = mfma_i8_k16(hb ? zero : mn, B);
             M2 = mfma_i8_k16(hb ? mn : zero, B);
+            mfma_result(M1);
+            mfma_result(M2);
         }
 #pragma unroll
         for (int i = 0; i < 16; i++) {
@@ -448,21 +456,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            u32x4 sm[16];                        // the rows' eight scales and eight mins
+#pragma unroll
+            for (int i = 0; i < 16; i++) sm[i] = *(const u32x4*)&s_sm[w][d_row(i, hb)][0];
 #pragma unroll
             for (int jj = 0; jj < 4; jj++) {
-                const v16i_k D0 = mfma_i8(and4(wq[jj], 0x0F0F0F0Fu), xb[2 * jj]);
-                const v16i_k D1 = mfma_i8(and4(shr4(wq[jj], 4), 0x0F0F0F0Fu), xb[2 * jj + 1]);
+                v16i_k D0 = mfma_i8(and4(wq[jj], 0x0F0F0F0Fu), xb[2 * jj]);
+                v16i_k D1 = mfma_i8(and4(shr4(wq[jj], 4), 0x0F0F0F0Fu), xb[2 * jj + 1]);
+                mfma_result(D0);
+                mfma_result(D1);
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const int row = d_row(i, hb);
-                    acc[i] += mul24(D0[i], (int)s_sm[w][row][2 * jj]) + mul24(D1[i], (int)s_sm[w][row][2 * jj + 1]);
+                    const uint32_t s2 = sm[i][jj >> 1] >> (16 * (jj & 1));
+                    acc[i] += mul24(D0[i], (int)(s2 & 0xffu)) + mul24(D1[i], (int)((s2 >> 8) & 0xffu));
                 }
             }
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int row = d_row(i, hb);
 #pragma unroll
-                for (int j = 0; j < 8; j++) mint[i] += mul24((int)s_sm[w][row][8 + j], xs8[j]);
+                for (int j = 0; j < 8; j++) mint[i] += mul24((int)((sm[i][2 + (j >> 2)] >> (8 * (j & 3))) & 0xffu), xs8[j]);
             }
         } else {
             // ql[128] = units 0-7, qh[64] = units 8-11, int8 scales = unit 12, d from the d stream
@@ -475,6 +487,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            u32x4 sm[16];                        // the rows' sixteen scales
+#pragma unroll
+            for (int i = 0; i < 16; i++) sm[i] = *(const u32x4*)&s_sm[w][d_row(i, hb)][0];
             // the superblock's activations, all eight requests in flight at once
             u32x4 xvs[8];
 #pragma unroll
@@ -496,12 +511,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                 // one 32 x 32 x 16 product per group
                 groups_to_k16(A);
                 groups_to_k16(xv);
-                const v16i_k D0 = mfma_i8_k16(uint2{A[0], A[1]}, uint2{xv[0], xv[1]});
-                const v16i_k D1 = mfma_i8_k16(uint2{A[2], A[3]}, uint2{xv[2], xv[3]});
+                v16i_k D0 = mfma_i8_k16(uint2{A[0], A[1]}, uint2{xv[0], xv[1]});
+                v16i_k D1 = mfma_i8_k16(uint2{A[2], A[3]}, uint2{xv[2], xv[3]});
+                mfma_result(D0);
+                mfma_result(D1);
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const int row = d_row(i, hb);
-                    acc[i] += mul24(D0[i], (int)(int8_t)s_sm[w][row][2 * m]) + mul24(D1[i], (int)(int8_t)s_sm[w][row][2 * m + 1]);
+                    const uint32_t s2 = sm[i][m >> 1] >> (16 * (m & 1));
+                    acc[i] += mul24(D0[i], (int)(int8_t)s2) + mul24(D1[i], (int)(int8_t)(s2 >> 8));
                 }
             }
         }

@@ -147,7 +147,8 @@ CPB_DEV void window_sums(u32x4* r, AFn a, float* S) {
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const v8i_mx B = {(int)r[t][0], (int)r[t][1], (int)r[t][2], (int)r[t][3], 0, 0, 0, 0};
-        const v4f_mx D = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a(t), B, v4f_mx{0, 0, 0, 0}, 0, 4, 0, 127, 0, 127);
+        v4f_mx D = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a(t), B, v4f_mx{0, 0, 0, 0}, 0, 4, 0, 127, 0, 127);
+        mfma_result(D);
         // lanes 0-15: blocks 0, 1 of row 16t + n; lanes 16-31: blocks 2, 3
         sa[t] = D[0] + D[1];
         sb[t] = D[2] + D[3];
