@@ -336,7 +336,9 @@ __global__ __launch_bounds__(64 * (1 + kPcProducers)) void k_router_exact_small(
     arrive();
 #pragma unroll
     for (int u = 0; u < 8; u++) v[u] = prod[0][u][lane];
-    for (; B * (k + 3) <= nb; k += 3) {
+    // (short of the end, so that the last three chunks' barriers are counted below:
+    // nch in all, as the producers')
+    for (; B * (k + 3) < nb; k += 3) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
 #pragma unroll

@@ -33,6 +33,8 @@ def check(L, cfg, X, family):
     (448, 64, 128, 4, 129),     # the first in short chunks
     (416, 64, 120, 2, 137),     # 13 blocks, half a chunk at the end, experts and tokens that are no whole groups
     (1568, 64, 128, 2, 133),    # more than the steps requested ahead
+    (768, 64, 128, 4, 129),     # a row that is whole rounds of the register sets, in short chunks
+    (1536, 64, 16, 2, 3),       # and in long ones
     (448, 64, 128, 4, 256),     # the last in short chunks
     (448, 64, 128, 4, 257),     # the first of the other kernel
 ])
