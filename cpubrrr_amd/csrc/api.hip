@@ -636,10 +636,15 @@ static int layer_grouped(cpb_moe_t* h, int layer, float* d_x, int n_tok, int app
     return 0;
 }
 
+// Whether n_tok tokens of a layer go through the batched kernels (else token by token)
+static bool takes_grouped(const cpb_moe_t* h, int layer, int n_tok) {
+    return n_tok > 1 && h->grouped && (h->mx ? h->layers[layer].mfma_exact : h->cfg.d <= 4096);
+}
+
 static int launch_direct(cpb_moe_t* h, int layer0, int n_layers, float* d_x, int n_tok, int apply_norm) {
     const auto& c = h->cfg;
     for (int l = layer0; l < layer0 + n_layers; l++) {
-        if (n_tok > 1 && h->grouped && (h->mx ? h->layers[l].mfma_exact : c.d <= 4096)) {
+        if (takes_grouped(h, l, n_tok)) {
             if (int r = layer_grouped(h, l, d_x, n_tok, apply_norm, nullptr, nullptr)) return r;
             continue;
         }
@@ -648,6 +653,9 @@ static int launch_direct(cpb_moe_t* h, int layer0, int n_layers, float* d_x, int
     }
     return 0;
 }
+
+constexpr int kGroupedKernels = 8;      // at most, of a layer through the batched path
+constexpr int kDirectKernels = 32;      // most kernels that a call launches without a graph
 
 int cpb_moe_forward_device(cpb_moe_t* h, int layer0, int n_layers, float* d_x, int n_tok, int apply_norm) {
     if (!h || !d_x) return fail(CPB_EINVAL, "NULL argument");
@@ -658,12 +666,16 @@ int cpb_moe_forward_device(cpb_moe_t* h, int layer0, int n_layers, float* d_x, i
         if (!h->layers[l].loaded) return fail(CPB_ESTATE, "layer %d not loaded", l);
     HIP_OK(hipSetDevice(h->device));
     // per-kernel timing needs one event pair per launch: run those directly.
-    // So does a single layer: a graph launch costs ~6 us between two calls that
-    // 3 to 8 queued kernels do not (one layer per call, per layer: Qwen decode
-    // 22.9 -> 18.3 us, gpt-oss 26.8 -> 21.4, 24 gpt-oss tokens 100.7 -> 95.2),
-    // and nothing is captured for a new x.  A stack of six layers in one call
-    // is faster as a graph (134 against 139 us).
-    if (h->timing || !h->use_graphs || n_layers == 1) return launch_direct(h, layer0, n_layers, d_x, n_tok, apply_norm);
+    // So does a single layer of few kernels: a graph launch costs ~6 us between
+    // two calls that 3 to 8 queued kernels do not (one layer per call, per layer:
+    // Qwen decode 22.9 -> 18.3 us, gpt-oss 26.8 -> 21.4, 24 gpt-oss tokens 100.7 ->
+    // 95.2), and nothing is captured for a new x.  Many kernels (a layer whose
+    // tokens go one by one: three each) are faster as a graph again, about 0.2 us a
+    // kernel: direct against graph 97.6 and 100.9 us at 24 kernels, 196.7 and 195.1
+    // at 48, 782 and 753 at 192, 6231 and 5974 at 1536 (d = d_ff = 480).  A stack of
+    // six layers in one call is faster as a graph too (134 against 139 us).
+    const bool few = n_layers == 1 && (takes_grouped(h, layer0, n_tok) ? kGroupedKernels : 3 * n_tok) <= kDirectKernels;
+    if (h->timing || !h->use_graphs || few) return launch_direct(h, layer0, n_layers, d_x, n_tok, apply_norm);
     // a caller capturing this stream into a graph of its own gets the
     // kernels themselves in that graph
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

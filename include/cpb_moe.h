@@ -133,8 +133,9 @@ int cpb_moe_forward(cpb_moe_t* h, int layer, float* x, int n_tok, int apply_norm
 /* Same on device memory, asynchronous on the handle's stream, over layers
  * [layer0, layer0 + n_layers).  d_x is a device pointer [n_tok][d].  The
  * layer loop of forward_worker (engine_gpt2.rs:767-930, MoE part only).
- * A single layer's kernels are launched directly; of calls over several
- * layers each distinct (layer0, n_layers, d_x, n_tok, apply_norm, stream) is
+ * A single layer's kernels are launched directly where they are few (all but
+ * the layers whose tokens go one by one, beyond 10 tokens); of other calls
+ * each distinct (layer0, n_layers, d_x, n_tok, apply_norm, stream) is
  * captured once into a HIP graph and replayed (at most 16 kept, least
  * recently used evicted).  If the stream is already being captured by the
  * caller, the kernels are launched into the caller's capture instead.      */
