@@ -272,6 +272,8 @@ int upload(float** dst, float* slot, const float* src, size_t n, hipStream_t s) 
 // then touch a few large pages instead of one small allocation per tensor
 // per layer, which keeps their address translations warm.
 size_t align64(size_t n) { return (n + 63) / 64 * 64; }
+// Whether a handle can take the batched path at all (the k-quant kernels go up to d = 4096)
+bool has_grouped(const cpb_moe_cfg& c) { return c.max_tokens > 1 && (c.wtype_gate_up == CPB_GGUF_MXFP4 || c.d <= 4096); }
 struct ParamSlots {
     size_t router_w, norm_w, router_b, gate_b, up_b, down_b, router_t, per_layer;
 };
@@ -285,7 +287,7 @@ ParamSlots param_slots(const cpb_moe_cfg& c) {
     p.gate_b = o; o += align64(ne * ff);
     p.up_b = o; o += align64(ne * ff);
     p.down_b = o; o += align64(ne * d);
-    p.router_t = o; o += c.max_tokens > 1 ? align64(cpb::router_t_rows(c.n_expert) * d) : 0;
+    p.router_t = o; o += has_grouped(c) ? align64(cpb::router_t_rows(c.n_expert) * d) : 0;
     p.per_layer = o;
     return p;
 }
@@ -477,7 +479,7 @@ int cpb_moe_create(const cpb_moe_cfg* cfg, int device, cpb_moe_t** out) {
     carve_decode(*cfg, h->dec_base, &h->b);
     if ((r = scratch_address(device, &h->noalloc_base))) return bail(r);
     if (h->mx && (r = dmalloc(&h->d_special, 1))) return bail(r);
-    h->grouped = T > 1;
+    h->grouped = has_grouped(*cfg);
     if (const char* v = getenv("CPB_GROUPED")) h->grouped = h->grouped && v[0] != '0';
     if (T > 1) {
         // grouped (batched) path: per-token and per-pair buffers; MXFP4 uses
@@ -581,7 +583,7 @@ int cpb_moe_load_layer_typed(cpb_moe_t* h, int layer, int gate_type, int up_type
             return r;
     }
     if ((r = upload(&L.router_w, base + ps.router_w, router_w, ne * d, h->stream))) return r;
-    if (c.max_tokens > 1) {
+    if (h->grouped) {
         L.router_t = base + ps.router_t;
         if (cpb::launch_router_transpose(L.router_w, L.router_t, c.n_expert, c.d, h->stream))
             return fail(CPB_ENODEV, "router transpose launch failed");
@@ -638,7 +640,7 @@ static int layer_grouped(cpb_moe_t* h, int layer, float* d_x, int n_tok, int app
 
 // Whether n_tok tokens of a layer go through the batched kernels (else token by token)
 static bool takes_grouped(const cpb_moe_t* h, int layer, int n_tok) {
-    return n_tok > 1 && h->grouped && (h->mx ? h->layers[layer].mfma_exact : h->cfg.d <= 4096);
+    return n_tok > 1 && h->grouped && (!h->mx || h->layers[layer].mfma_exact);
 }
 
 static int launch_direct(cpb_moe_t* h, int layer0, int n_layers, float* d_x, int n_tok, int apply_norm) {
@@ -732,10 +734,11 @@ int cpb_moe_grouped_sums(cpb_moe_t* h, int layer, float* x, int n_tok, int apply
                          int32_t* dn_sums) {
     if (!h || !x || !gu_sums || !dn_sums) return fail(CPB_EINVAL, "NULL argument");
     const auto& c = h->cfg;
-    if (!h->grouped) return fail(CPB_EINVAL, "grouped path needs max_tokens > 1");
+    const bool wide = !h->mx && c.d > 4096;
+    if (c.max_tokens < 2 || (!h->grouped && !wide)) return fail(CPB_EINVAL, "grouped path needs max_tokens > 1");
     if (layer < 0 || layer >= c.n_layer || !h->layers[layer].loaded) return fail(CPB_ESTATE, "layer %d not loaded", layer);
     if (h->mx && !h->layers[layer].mfma_exact) return fail(CPB_EINVAL, "layer %d has e8m0 scales outside [32, 254]", layer);
-    if (!h->mx && c.d > 4096) return fail(CPB_EINVAL, "k-quant grouped path takes d <= 4096");
+    if (wide) return fail(CPB_EINVAL, "k-quant grouped path takes d <= 4096");
     if (n_tok < 2 || n_tok > c.max_tokens) return fail(CPB_EINVAL, "n_tok=%d outside [2, max_tokens=%d]", n_tok, c.max_tokens);
     HIP_OK(hipSetDevice(h->device));
     const size_t d = c.d, np = (size_t)n_tok * c.top_k;

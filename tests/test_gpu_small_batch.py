@@ -88,3 +88,18 @@ def test_mxfp4_tiles(gpu, d, dff, ne, k, n_tok):
     L = synth.gptoss_layer(d, dff, ne, k, seed=24, zipf=1.1)
     X = np.stack([synth.token(d, 24, i) for i in range(n_tok)])
     check(L, MoeConfig.gptoss(d=d, n_expert=ne, top_k=k, d_ff=dff, max_tokens=n_tok), X, "gptoss")
+
+
+@pytest.mark.parametrize("d,kept", [(4096, True), (8192, False)])
+def test_router_copy_only_for_the_batched_path(gpu, d, kept):
+    """The transposed router copy (4 n_expert d bytes a layer) belongs to handles that can take the batched path."""
+    print(f"case router copy d={d}", flush=True)
+    import torch
+    ne, layers = 256, 32
+    used = []
+    for tokens in (1, 1, 2):                         # the first handle also brings in the library's code
+        before = torch.cuda.mem_get_info()[0]
+        with MoeBlock(MoeConfig.qwen3(d=d, n_expert=ne, top_k=8, d_ff=256, n_layer=layers, max_tokens=tokens)):
+            used.append(before - torch.cuda.mem_get_info()[0])
+    copy = 4 * ne * d * layers
+    assert (used[2] - used[1] >= copy // 2) == kept, (used, copy)
