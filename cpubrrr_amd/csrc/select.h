@@ -18,10 +18,9 @@ namespace cpb {
 // candidates whose exact serial logits are computed side by side (the decode
 // kernels' LDS budget)
 constexpr int kExactGroup = 4;
-// LDS floats per candidate's product row: d plus the chain's look-ahead slack
-// (64 floats), a multiple of 4 (16-byte reads) that spreads the chain lanes
-// over the banks
-CPB_DEV_HOST_INLINE int exact_stride(int d) { return d + 68; }
+// LDS floats per candidate's product row: a multiple of 4 (16-byte reads) that
+// spreads the chain lanes over the banks (d is a multiple of 32)
+CPB_DEV_HOST_INLINE int exact_stride(int d) { return d + 4; }
 // acc += v in order, 32 products, fp32 round to nearest (the reference's
 // serial chain)
 CPB_DEV float serial_add32(const f32x4 (&v)[8], float acc) {
