@@ -55,6 +55,8 @@ def test_mxfp4_small_batches(gpu, d, dff, ne, k, n_tok):
     (1280, 768, 16, 4, 16, 14, False),      # four pairs per expert: the last size of the few-token kernels
     (1280, 768, 16, 4, 17, 14, False),      # the first of the matrix-core tiles
     (512, 2048, 16, 2, 4, 14, False),       # d_ff beyond the few-token down kernel
+    (4096, 1536, 8, 2, 7, 14, False),       # the few-token kernels at their widest: 512 threads, more than 64 KB of LDS
+    (4096, 1536, 8, 4, 8, 12, True),        # and with full tiles
 ])
 def test_kq_small_batches(gpu, d, dff, ne, k, n_tok, down, same):
     print(f"case kq small batch d={d} dff={dff} ne={ne} k={k} n_tok={n_tok} down={down}", flush=True)
