@@ -217,8 +217,8 @@ def _host_info() -> dict:
 def cpu_baseline(host_layers, c, budget_s: float) -> dict:
     """Oracle (C restatement of the reference path, OpenMP over rows) on the
     host's cores, over the first layers of the same workload: threaded over
-    every core this process may use (capped by OMP_NUM_THREADS, the host's
-    per-GPU CPU share on the GPU boxes), and single-threaded."""
+    every core this process may use (capped by OMP_NUM_THREADS, the
+    per-GPU share of a node's CPUs), and single-threaded."""
     import numpy as np
     from oracle import oracle as O
     from cpubrrr_amd import synth
@@ -612,7 +612,7 @@ def main() -> int:
                     help="also run one plain device copy of this many MiB (HBM-traffic counter calibration)")
     args = ap.parse_args()
     if args.gpus != 1:
-        print(f"bench.py measures one GPU only: this build has no multi-GPU path (asked for --gpus {args.gpus}); "
+        print(f"bench.py measures one GPU only: there is no multi-GPU path (asked for --gpus {args.gpus}); "
               "run with --gpus 1", file=sys.stderr)
         return 2
 

@@ -379,8 +379,9 @@ int launch_router_transpose(const float* w, float* out, int ne, int d, hipStream
 // rounds of a wave maximum, the lowest index by ballot.  A NaN ranks last (a
 // strict comparison never lets one in), as -inf.
 // Bound by the rounds' chain in the wave, so four tokens share a workgroup to
-// put all of them in flight at once: 512 tokens x 32 experts 4.8 us, where
-// decode's selector with its intervals and certificate took 22.
+// put all of them in flight at once (kernel traces, against decode's selector
+// with its intervals and certificate): 512 tokens x 32 experts 6.2 -> 5.0 us, 2049
+// x 128 22 -> 5.
 struct TokenLogits {
     float v[4];
 };
@@ -646,8 +647,11 @@ CPB_DEV void split_pair(const u32x4& v, u32x4& x, u32x4& y) {
 // 61 ns per block and tile against 28 of matrix-core and 27 of VALU work: two,
 // three and four waves per SIMD all ran at that rate).  512 tokens x 32
 // experts: gate/up 161 -> 149 us, down 87 -> 76; 2049 x 128: 574 -> 496 and
-// 298 -> 255.  Now reads, fmas and products take about the same time.  Per
-// block, D = A(rows) x B(tokens) on the matrix cores and acc = fma(D, xsb, acc)
+// 298 -> 255 (kernel traces of one layer called again and again).  Now VALU
+// issue comes first: by the counters at 512 tokens it takes 56 % of the
+// gate/up's time (30 instructions per MFMA: 16 fmas, 4 exchanges of split_pair, 2
+// chain adds, the MFMA and an address in the loop, 5 before and after it), the
+// matrix cores 30 % and the LDS reads about as much.  Per block, D = A(rows) x B(tokens) on the matrix cores and acc = fma(D, xsb, acc)
 // in block order, in two chains per k-part (its sub-parts, as the decode
 // kernels' two wavefronts per k-part), the chains added to the total in order.
 //

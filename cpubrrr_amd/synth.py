@@ -1,5 +1,5 @@
 """Synthetic workloads of the bench configs, generated through the C ABI
-(cpb_synth_*) so the host here, the GPU box and every test produce identical
+(cpb_synth_*) so every host and every test produce identical
 bytes from (seed, layer).
 
 Distributions:

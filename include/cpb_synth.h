@@ -1,7 +1,7 @@
 /* cpb_synth.h -- deterministic synthetic weights and activations.
  *
- * Generates the bench workloads' tensors from (seed, stream) so that the
- * host here, the GPU box and every test produce identical bytes.  Counter
+ * Generates the bench workloads' tensors from (seed, stream) so that
+ * every host and every test produce identical bytes.  Counter
  * based (splitmix64 finaliser of key + index), so any slice can be generated
  * independently and in parallel.  Host-only; no GPU calls.
  *

@@ -4,7 +4,7 @@
 
 gcc, -O3, -ffp-contract=off (the reference never contracts a*b+c; its NEON
 fmas are written out as fmaf), OpenMP over independent rows.  -march is a
-portable x86-64-v3 so the library built here also runs on the GPU box's host.
+portable x86-64-v3 so that the library runs on any such host.
 """
 from __future__ import annotations
 
