@@ -3,8 +3,8 @@
 The hardware does not hold back a vector or memory instruction that uses an
 MFMA's result too early: the instructions between have to take up enough issue
 states (the product's passes + 3, one more on gfx950 from 4 passes on).  The
-compiler pads to that, but counts every s_waitcnt as a state, and one that is
-already satisfied takes none.  So the states are counted here without waits and
+compiler pads to that, but counts every s_waitcnt as a state, and by what was
+seen one that is already satisfied takes none.  So the states are counted here without waits and
 barriers, over every path, in the assembly of each source that has products,
 built with the library's own flags.
 """
